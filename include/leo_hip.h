@@ -219,7 +219,7 @@ typedef struct LeoKernelStats {
      * the weight unchanged, bit for bit). */
     uint64_t learning_slots;
     /* Delivery buckets of more than 8 entries in one tick, folded by a whole
-     * wave after a sort: ranked in registers (up to 128 entries) or radix
+     * wave after a sort: ranked in LDS (up to 256 entries) or radix
      * sorted through the target's shadow range. */
     uint64_t deep_register_folds;
     uint64_t deep_radix_folds;

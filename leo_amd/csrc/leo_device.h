@@ -73,8 +73,9 @@ inline __host__ __device__ size_t window_bytes(uint32_t neurons_per_block) {
 constexpr uint32_t kStageRowFloats = 33;
 constexpr size_t kStageBytes = 64 * kStageRowFloats * 4;
 
-// Radix counts of a wave's deep-bucket sort, after its window: the current
-// pass's 256 scatter offsets and the next pass's 256 counts.
+// A wave's deep-bucket stage, after its window: 256 ranked entries (value,
+// branch), or the radix sort's counts (the current pass's 256 scatter offsets
+// and the next pass's 256 counts).
 constexpr size_t kDeepHistBytes = 2 * 256 * 4;
 
 // Per-wave share of the dynamic LDS: the phase-2 window (reused by the
@@ -160,7 +161,7 @@ struct StepRecord {
     float neural_max;
     float neural_sum;
     float neural_target;
-    uint32_t deep_folds;        // buckets of more than 8 deliveries: ranked in registers (low 16 bits),
+    uint32_t deep_folds;        // buckets of more than 8 deliveries: ranked (low 16 bits),
                                 // radix-sorted (high 16 bits)
 };
 
@@ -413,11 +414,11 @@ inline __host__ __device__ uint32_t edge_branch(uint32_t e) { return e >> (kEdge
 // bucket by delivery key (delay class, the emitting neuron's active rank, its
 // synapse slot; or class 4 and the input slot), which is unique per entry, so
 // each branch's accumulator receives its values in the reference's delivery
-// order (runtime.rs:605-639). Up to kDeepRegisterEntries entries are ranked in
-// registers; larger buckets, which only targets of that capacity can have, go
+// order (runtime.rs:605-639). Up to kDeepRankEntries entries are ranked in
+// LDS; larger buckets, which only targets of that capacity can have, go
 // through an LSD radix sort with 8-bit digits between the bucket and the
 // target's shadow range, on a compacted key of the significant fields.
-constexpr uint32_t kDeepRegisterEntries = 128;
+constexpr uint32_t kDeepRankEntries = 256;  // four per lane
 constexpr uint32_t kDeepMaxPasses = 8;
 struct DeepSortPlan {
     uint32_t rank_bits;                   // bits of the rank field (active rank or input slot)

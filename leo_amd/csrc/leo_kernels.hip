@@ -1227,13 +1227,106 @@ struct DeepArray {
 
 constexpr uint32_t kDeepTiles = 8;  // 64-entry tiles a lane has in flight
 
+// The ranks of K entries per lane among `cnt` keys in LDS (distinct, padded to
+// a multiple of four with the largest key): the number of smaller keys. Four
+// keys per 16-byte LDS read (the same address on every lane), two instructions
+// per key and entry.
+template <uint32_t K, class Key>
+__device__ __forceinline__ void deep_ranks(const Key* keys, uint32_t cnt, const Key (&mine)[4], uint32_t (&rank)[4]) {
+    for (uint32_t q = 0; q < cnt; q += 4) {
+        Key other[4];
+#pragma unroll
+        for (uint32_t x = 0; x < 4; ++x) other[x] = keys[q + x];
+#pragma unroll
+        for (uint32_t k = 0; k < K; ++k) {
+#pragma unroll
+            for (uint32_t x = 0; x < 4; ++x) rank[k] += other[x] < mine[k] ? 1u : 0u;
+        }
+    }
+}
+
+// The branch sums of a bucket of at most kDeepRankEntries entries, by the
+// whole wave: lane b < 4 starts from branch b's accumulator and returns it
+// with the branch's values added in delivery order. Up to four entries per
+// lane are ranked against all keys in LDS (`stage`, 2 KB), written to their
+// places there, and read back in order; an entry of another branch adds -0.0,
+// which leaves every sum as it is, so the chain is one add per entry. Sort
+// keys of at most 32 bits (all but enormous models) are compared as words.
+// Latency-bound: the wave that owns a hub ends the lane's phase. With 131,072
+// units and power-law targets (1,876 deliveries a step, hubs of 70-200) a
+// frozen step took 22.6 us with ranks counted and entries broadcast through
+// lane reads up to 128 entries and a radix sort above, and takes 17.1 us; at
+// 256 entries the ranking is ~1,000 compares a lane, still under the radix
+// sort's three passes over memory, and four entries per lane is what the 2 KB
+// stage holds.
+__device__ __forceinline__ float deep_ranked_sum(const KernelArgs& a, const uint64_t LEO_GLOBAL* set_base,
+                                                 const DeepArray& bucket, uint32_t cnt, uint32_t* stage, float acc) {
+    const uint32_t lane = __lane_id();
+    const __amdgpu_buffer_rsrc_t entries = record_rsrc(set_base, 16, 0xffffffffu);
+    f32x4 e[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t p = k * kWaveSize + lane;
+        e[k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (p < cnt) e[k] = ld16_record(entries, static_cast<uint32_t>(bucket.at(p)), 0);
+    }
+    const uint32_t padded = (cnt + 3) & ~3u;
+    uint32_t rank[4] = {0, 0, 0, 0};
+    uint64_t key[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+        key[k] = (static_cast<uint64_t>(__float_as_uint(e[k].y)) << 32) | __float_as_uint(e[k].x);
+    if (a.deep.rank_bits + a.deep.slot_bits + 3 <= 32) {
+        uint32_t word[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t p = k * kWaveSize + lane;
+            word[k] = p < cnt ? static_cast<uint32_t>(deep_sort_key(key[k], a.deep.rank_bits, a.deep.slot_bits)) : ~0u;
+            if (p < padded) stage[p] = word[k];
+        }
+        wave_sync();
+        if (cnt <= kWaveSize) deep_ranks<1>(stage, cnt, word, rank);
+        else if (cnt <= 2 * kWaveSize) deep_ranks<2>(stage, cnt, word, rank);
+        else deep_ranks<4>(stage, cnt, word, rank);
+    } else {
+        uint64_t* wide = reinterpret_cast<uint64_t*>(stage);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t p = k * kWaveSize + lane;
+            if (p >= cnt) key[k] = ~0ULL;
+            if (p < padded) wide[p] = key[k];
+        }
+        wave_sync();
+        deep_ranks<4>(wide, cnt, key, rank);
+    }
+    wave_sync();
+    // (value, branch) pairs in delivery order, the padding of no branch
+    uint2* sorted = reinterpret_cast<uint2*>(stage);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t p = k * kWaveSize + lane;
+        if (p < cnt) sorted[rank[k]] = make_uint2(__float_as_uint(e[k].z), __float_as_uint(e[k].x) & 3u);
+        else if (p < padded) sorted[p] = make_uint2(0u, kWaveSize);
+    }
+    wave_sync();
+    const uint4* pairs = reinterpret_cast<const uint4*>(stage);
+    for (uint32_t q = 0; q < padded / 2; q += 2) {
+        const uint4 u = pairs[q], w = pairs[q + 1];
+        acc += u.y == lane ? __uint_as_float(u.x) : -0.0f;
+        acc += u.w == lane ? __uint_as_float(u.z) : -0.0f;
+        acc += w.y == lane ? __uint_as_float(w.x) : -0.0f;
+        acc += w.w == lane ? __uint_as_float(w.z) : -0.0f;
+    }
+    wave_sync();  // the stage is free for the wave's next deep bucket
+    return acc;
+}
+
 // fold_drive of a neuron with more than 8 deliveries, by the whole wave (all
 // lanes active, n uniform): the bucket is sorted by delivery key -- ranked in
-// registers up to kDeepRegisterEntries entries, else by an LSD radix sort
-// between the bucket and the target's shadow range with the histogram in
-// `hist` (256 words of LDS) -- and every lane adds the entries in that order
-// (uniform values, so every lane holds the same sums). Lane 0 writes the
-// state.
+// LDS up to kDeepRankEntries entries (deep_ranked_sum), else by an LSD radix
+// sort between the bucket and the target's shadow range with the histogram in
+// `hist` (512 words of LDS) -- and its entries are added in that order
+// (uniform sums, so every lane holds them). Lane 0 writes the state.
 __device__ float deep_fold(const StepCtx& c, uint32_t n, float pi, uint32_t set, bool post_pending, bool* refractory,
                            uint32_t* hist) {
     const KernelArgs& a = *c.a;
@@ -1277,35 +1370,12 @@ __device__ float deep_fold(const StepCtx& c, uint32_t n, float pi, uint32_t set,
         b3 = br == 3 ? b3 + v : b3;
     };
     DeepArray bucket{set_base, overflow, n, true};
-    if (cnt <= kDeepRegisterEntries) {
-        // two entries per lane; rank = number of smaller keys (keys unique)
-        uint64_t k0 = ~0ULL, k1 = ~0ULL;
-        uint32_t v0 = 0, v1 = 0;
-        if (lane < cnt) {
-            const uint64_t at = bucket.at(lane);
-            k0 = ld(&set_base[2 * at]);
-            v0 = static_cast<uint32_t>(ld(&set_base[2 * at + 1]));
-        }
-        if (lane + kWaveSize < cnt) {
-            const uint64_t at = bucket.at(lane + kWaveSize);
-            k1 = ld(&set_base[2 * at]);
-            v1 = static_cast<uint32_t>(ld(&set_base[2 * at + 1]));
-        }
-        uint32_t r0 = 0, r1 = 0;
-        for (uint32_t q = 0; q < cnt; ++q) {
-            const uint64_t kq = readlane_u64(q < kWaveSize ? k0 : k1, q & (kWaveSize - 1));
-            r0 += kq < k0 ? 1u : 0u;
-            r1 += kq < k1 ? 1u : 0u;
-        }
-        for (uint32_t r = 0; r < cnt; ++r) {
-            const uint64_t m0 = __ballot(lane < cnt && r0 == r);
-            const uint64_t m1 = __ballot(lane + kWaveSize < cnt && r1 == r);
-            const bool first = m0 != 0;
-            const uint32_t src = static_cast<uint32_t>(__ffsll(static_cast<long long>(first ? m0 : m1)) - 1);
-            const uint32_t key_lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(first ? k0 : k1), static_cast<int>(src));
-            const uint32_t bits = __builtin_amdgcn_readlane(first ? v0 : v1, static_cast<int>(src));
-            add(key_lo, bits);
-        }
+    if (cnt <= kDeepRankEntries) {
+        const float acc = deep_ranked_sum(a, set_base, bucket, cnt, hist, lane < 2 ? (lane == 0 ? b0 : b1) : (lane == 2 ? b2 : b3));
+        b0 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(acc), 0));
+        b1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(acc), 1));
+        b2 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(acc), 2));
+        b3 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(acc), 3));
     } else {
         // LSD radix sort, 8-bit digits; each pass reads its source in order
         // (kDeepTiles tiles of 64 entries in flight per lane), counts the
@@ -1428,9 +1498,9 @@ __device__ float deep_fold(const StepCtx& c, uint32_t n, float pi, uint32_t set,
     }
     if (lane == 0) {
         if (c.tally)
-            c.tally[cnt <= kDeepRegisterEntries ? kTDeepRegister : kTDeepRadix] += 1u;
+            c.tally[cnt <= kDeepRankEntries ? kTDeepRegister : kTDeepRadix] += 1u;
         else
-            atomicAdd(counter_word(c, c.part, kCDeep, tick), cnt <= kDeepRegisterEntries ? 1u : 0x10000u);
+            atomicAdd(counter_word(c, c.part, kCDeep, tick), cnt <= kDeepRankEntries ? 1u : 0x10000u);
         if (e > 0) {
             (*nf(d, n, kNFatigue)) = fat;
             (*nf(d, n, kNAdapt0)) = ad0;

@@ -1781,7 +1781,7 @@ void upload_topology(LeoHipRuntime* h, const LeoModelView& m) {
     std::vector<uint64_t> shadow(z.n + 1, 0);
     for (uint64_t n = 0; n < z.n; ++n) {
         const uint64_t need = cap[n] + row_max[n];
-        shadow[n + 1] = shadow[n] + (need > kDeepRegisterEntries ? need : 0);
+        shadow[n + 1] = shadow[n] + (need > kDeepRankEntries ? need : 0);
     }
     h->z.shadow_total = shadow[z.n];
     Layout l;
