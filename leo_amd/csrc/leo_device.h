@@ -67,22 +67,15 @@ inline __host__ __device__ size_t window_bytes(uint32_t neurons_per_block) {
     return (c * 12 + kGroupBlocks * 8 + (kGroupBlocks + 1) * 4 + kGroupBlocks * 8 + words * 8 + 15) / 16 * 16;
 }
 
-// Learning-signal row staging of one wave: 64 output rows, one 128-byte line
-// (32 floats) of each at a time, rows padded to 33 floats (conflict-free
-// column reads).
-constexpr uint32_t kStageRowFloats = 33;
-constexpr size_t kStageBytes = 64 * kStageRowFloats * 4;
-
 // A wave's deep-bucket stage, after its window: 256 ranked entries (value,
 // branch), or the radix sort's counts (the current pass's 256 scatter offsets
 // and the next pass's 256 counts).
 constexpr size_t kDeepHistBytes = 2 * 256 * 4;
 
-// Per-wave share of the dynamic LDS: the phase-2 window (reused by the
-// learning-signal staging), then the deep-bucket histogram.
+// Per-wave share of the dynamic LDS: the phase-2 window, then the deep-bucket
+// stage.
 inline __host__ __device__ size_t wave_window_bytes(uint32_t neurons_per_block) {
-    const size_t w = window_bytes(neurons_per_block);
-    return ((w > kStageBytes ? w : kStageBytes) + 15) / 16 * 16;
+    return window_bytes(neurons_per_block);
 }
 inline __host__ __device__ size_t wave_lds_bytes(uint32_t neurons_per_block) {
     return wave_window_bytes(neurons_per_block) + kDeepHistBytes;

@@ -452,7 +452,6 @@ constexpr uint32_t kStepChunk = 64;
 struct alignas(16) StepShared {
     float err[kOutStride];                                      // errors / logits
     float aux[kOutStride + kThreads];                           // exps, latent, gradient
-    uint32_t queue[kWavesPerGroup][2 * kWaveSize];              // per-wave destination queue
     uint32_t scan[kThreads];
     unsigned long long red[kWavesPerGroup];
     float redf[kWavesPerGroup];
@@ -3011,102 +3010,109 @@ __device__ __forceinline__ void phase_post(const StepCtx& c, const StepParams& s
 }
 
 // ---------------------------------------------------------------------------
-// Phase 5: learning destinations and signals (runtime.rs:1214-1263). Each wave
-// claims destinations, queues them, and computes their serial 257-term dot
-// products 64 at a time from output rows staged through LDS (coalesced row
-// loads).
+// Phase 5: learning signals of the claimed destinations (runtime.rs:1214-1263),
+// the serial 257-term dot products of their output rows with the errors.
 // ---------------------------------------------------------------------------
-// Device-scope 16-byte loads through a buffer resource (cache policy sc1: the
-// load misses the CU's L1 like ld()); the resource is wave-uniform and covers
-// `bytes` from `base` (loads beyond it return 0).
-// Serial 257-term dot of one output row with the errors, in output order
-// (runtime.rs:1245-1250).
-// Learning signals of up to 64 destinations, one per lane (`dst` on lanes
-// below `count`; every lane of the wave calls): the output rows are streamed
-// through the wave's LDS stage one 128-byte line at a time, 8 whole lines per
-// load instruction, with the next two lines in flight while the current one
-// is summed; each lane then adds its row's 257 products in the reference's
-// order (runtime.rs:1214-1263).
-__device__ __forceinline__ float signal_rows(__amdgpu_buffer_rsrc_t rows, uint32_t dst, uint32_t count, const float* err,
-                                             float* stage) {
-    constexpr uint32_t kLines = kEndIndex / 32;  // 128-byte lines before the end-class weight
-    const uint32_t lane = __lane_id();
-    const uint32_t seg = lane & 7, sub = lane >> 3;
-    // this lane loads 16 bytes of rows sub, 8 + sub, ..., 56 + sub
-    uint32_t row_of[8];
-    bool live[8];
+// A batch is eight destinations, whose output rows a wave loads whole in one
+// round (eight 16-byte loads per lane, one 128-byte line of a row per eight
+// lanes) and sums in registers. The sum of a row is serial in output order
+// (runtime.rs:1245-1250), so its accumulator travels: a row of sixteen lanes
+// is a ring for two output rows, A and B, half a turn apart; at stage k
+// (outputs 4k to 4k+3) lane k % 16 adds its four products of A, lane
+// (k + 8) % 16 those of B, and a rotation by one lane, part of the stage's
+// first add, hands both on. Lanes 0-7 hold the even lines of A and the odd
+// lines of B, lanes 8-15 the others: every lane then takes line l from
+// register l. (The other lanes' sums at a stage are no row's and are not
+// used.) A batch costs one memory round and ~300 instructions whatever the
+// destinations number, and batches are dealt over every wave of the lane.
+// With 64 rows a batch, staged through LDS line by line, a few hundred to a
+// thousand destinations occupied 8 to 23 waves of 64 to 128 for four memory
+// rounds. Post phase with signals, per step: 16,384 units, 506 destinations,
+// 64 waves: 7.2 us then, 4.8 now; a million units, ~1,000 destinations, 32
+// workgroups: 29% less; a 32-lane story pass at 131,072 units 17.8 -> 15.9 ms
+// (with the deep buckets' 1.1 ms).
+constexpr uint32_t kSignalRows = 8;
+constexpr uint32_t kSignalLines = kEndIndex / 32;  // 128-byte lines before the end-class weight
+
+struct SignalRows {
+    f32x4 line[kSignalLines];
+    float tail;        // the end-class weight of the row this lane ends with
+    uint32_t dst_end;  // and that row's destination
+    bool live_end;
+};
+__device__ __forceinline__ uint32_t swap_halves(uint32_t v) {  // lanes 0-7 and 8-15 of each sixteen exchanged
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xf, 0xf, false));
+}
+// `dst`: the destination of row lane / 8 (0 past the batch's end, `live` false).
+__device__ __forceinline__ void load_signal_rows(SignalRows& r, __amdgpu_buffer_rsrc_t rows, uint32_t dst, bool live) {
+    const uint32_t seg = __lane_id() & 7u;
+    const uint32_t other = swap_halves(dst);
 #pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        const uint32_t row = 8 * k + sub;
-        live[k] = row < count;
-        row_of[k] = static_cast<uint32_t>(__shfl(static_cast<int>(dst), static_cast<int>(row)));
-    }
-    const float tail = lane < count ? ld4_record(rows, dst, 4 * kEndIndex) : 0.0f;
-    // two lines in flight (even lines in v, odd lines in w; the unrolled loop
-    // names the buffers statically, so no register copy waits for a load)
-    static_assert(kLines % 2 == 0, "lines are taken in pairs");
-    f32x4 v[8], w[8];
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        v[k] = live[k] ? ld16_record(rows, row_of[k], seg * 16) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        w[k] = live[k] ? ld16_record(rows, row_of[k], seg * 16 + 128) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    for (uint32_t l = 0; l < kSignalLines; ++l) r.line[l] = ld16_record(rows, (l & 1) ? other : dst, l * 128 + seg * 16);
+    r.tail = ld4_record(rows, other, 4 * kEndIndex);
+    r.dst_end = other;
+    r.live_end = swap_halves(live ? 1u : 0u) != 0;
+}
+// The serial sums; lanes 7 and 15 of each sixteen return those of their dst_end.
+__device__ __forceinline__ float sum_signal_rows(const SignalRows& r, const f32x4 (&err)[kSignalLines], float err_end) {
     float acc = 0.0f;
+    auto rotate = [](float v) {  // from the lane below, within sixteen
+        return __uint_as_float(static_cast<uint32_t>(
+            __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0x121, 0xf, 0xf, false)));
+    };
 #pragma unroll
-    for (uint32_t line = 0; line < kLines; ++line) {
-        f32x4(&cur)[8] = (line & 1) ? w : v;
-        wave_sync();
+    for (uint32_t l = 0; l < kSignalLines; ++l) {
+        const float p0 = r.line[l].x * err[l].x, p1 = r.line[l].y * err[l].y;
+        const float p2 = r.line[l].z * err[l].z, p3 = r.line[l].w * err[l].w;
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) {
-            float* st = stage + (8 * k + sub) * kStageRowFloats + seg * 4;
-            st[0] = cur[k].x;
-            st[1] = cur[k].y;
-            st[2] = cur[k].z;
-            st[3] = cur[k].w;
-        }
-        wave_sync();
-        if (line + 2 < kLines) {
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k)
-                cur[k] = live[k] ? ld16_record(rows, row_of[k], seg * 16 + (line + 2) * 128)
-                                 : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-        if (lane < count) {
-            const float* r = stage + lane * kStageRowFloats;
-            const float* e = err + line * 32;
-#pragma unroll
-            for (uint32_t o = 0; o < 32; ++o) acc += r[o] * e[o];
+        for (uint32_t s = 0; s < 8; ++s) {
+            acc = rotate(acc) + p0;
+            acc += p1;
+            acc += p2;
+            acc += p3;
         }
     }
-    acc += tail * err[kEndIndex];
-    return acc;
+    return acc + r.tail * err_end;
 }
 
-// The listed destinations' signals (runtime.rs:1245-1250), 64 at a time per
-// wave, the batches dealt round-robin over every wave of the lane.
+// The listed destinations' signals, the batches dealt round-robin over every
+// wave of the lane, the next batch's rows loaded while one is summed.
 __device__ __forceinline__ void phase_signals(const StepCtx& c, StepShared& sh) {
     const LaneDesc& d = c.d;
-    const LeoConfig& cfg = c.a->cfg;
-    // one round: the errors, the destination count and this wave's first
-    // batch of the list (read before the count is known; entries past it are
-    // masked below)
-    const uint32_t wave = wave_index(), lane = __lane_id();
-    // batches of 64 destinations dealt to the workgroups in turn
-    const uint32_t waves = c.P * kWavesPerGroup, b0 = wave * c.P + c.part;
-    const uint32_t N = cfg.neuron_count;
+    // one round: the errors, the destination count and this wave's first two
+    // batches of the list (read before the count is known; entries past it
+    // are masked below)
+    const uint32_t lane = __lane_id(), sub = lane >> 3;
+    const uint32_t stride = c.P * kWavesPerGroup * kSignalRows;
+    const uint32_t N = c.a->cfg.neuron_count;
+    uint32_t at = (wave_index() * c.P + c.part) * kSignalRows + sub;
     const uint32_t count = ld(&c.ctl->dest_count);
-    const uint32_t first_at = b0 * kWaveSize + lane;
-    const uint32_t first_dst = first_at < N ? ld(&d.dest_list[first_at]) : 0u;
+    uint32_t dst = at < N ? ld(&d.dest_list[at]) : 0u;
+    uint32_t next = at + stride < N ? ld(&d.dest_list[at + stride]) : 0u;
     for (uint32_t o = threadIdx.x; o < kOutputs; o += kThreads) sh.err[o] = ld(&d.errors[o]);
     __syncthreads();
+    if (at - sub >= count) return;  // wave-uniform
+    f32x4 err[kSignalLines];
+#pragma unroll
+    for (uint32_t l = 0; l < kSignalLines; ++l)
+        err[l] = reinterpret_cast<const f32x4*>(sh.err)[l * 8 + (lane & 7u)];
+    const float err_end = sh.err[kEndIndex];
     // rows addressed by index (N records of kOutStride floats)
     const __amdgpu_buffer_rsrc_t rows = record_rsrc(d.p.out_w, kOutStride * 4, N);
-    float* stage = reinterpret_cast<float*>(step_lds + static_cast<size_t>(wave) * wave_lds_bytes(cfg.neurons_per_block));
-    for (uint32_t b = b0; b * kWaveSize < count; b += waves) {
-        const uint32_t n = min(kWaveSize, count - b * kWaveSize);
-        const uint32_t dst = lane < n ? (b == b0 ? first_dst : ld(&d.dest_list[b * kWaveSize + lane])) : 0u;
-        const float sig = signal_rows(rows, dst, n, sh.err, stage);
-        if (lane < n) d.learning_signal[dst] = sig;
+    SignalRows cur;
+    load_signal_rows(cur, rows, at < count ? dst : 0u, at < count);
+    while (true) {
+        at += stride;
+        const bool more = at - sub < count;  // wave-uniform
+        SignalRows ahead = cur;
+        if (more) {
+            load_signal_rows(ahead, rows, at < count ? next : 0u, at < count);
+            next = at + stride < N ? ld(&d.dest_list[at + stride]) : 0u;
+        }
+        const float sig = sum_signal_rows(cur, err, err_end);
+        if ((lane & 7u) == 7u && cur.live_end) d.learning_signal[cur.dst_end] = sig;
+        if (!more) break;
+        cur = ahead;
     }
 }
 
