@@ -57,14 +57,11 @@ constexpr uint32_t kFixedEntries = 4;
 inline __host__ __device__ uint32_t window_capacity(uint32_t neurons_per_block) {
     return neurons_per_block > 256 ? neurons_per_block : 256;
 }
-// Per-wave bytes of the window: u64 keys and u32 entries (capacity each),
-// block cutoff keys (G), block starts (G+1), block candidate counts and
-// staged winner offsets (G each), and
-// the group's bitmap words with their list positions (64*kWordsPerLane each).
+// Per-wave bytes of the window: touched neurons, then the candidates' u64 keys,
+// blocks and order by block (capacity each), and the group's block starts.
 inline __host__ __device__ size_t window_bytes(uint32_t neurons_per_block) {
     const size_t c = window_capacity(neurons_per_block);
-    const size_t words = 64 * kWordsPerLane;
-    return (c * 12 + kGroupBlocks * 8 + (kGroupBlocks + 1) * 4 + kGroupBlocks * 8 + words * 8 + 15) / 16 * 16;
+    return (c * 20 + (kGroupBlocks + 1) * 4 + 15) / 16 * 16;
 }
 
 // A wave's deep-bucket stage, after its window: 256 ranked entries (value,

@@ -434,10 +434,6 @@ __device__ __forceinline__ uint32_t next_pow2(uint32_t v) {
     return p;
 }
 
-// Window key of a neuron whose deep bucket the wave folds after the others
-// (above every selection key, whose high word is at most 0xfffffffe).
-constexpr uint64_t kDeepPending = ~1ULL;
-
 // Selection key: ascending order == (activation desc, rotated tie key asc)
 // (runtime.rs:987-1009); activation > 0 so its bit pattern is monotone.
 __device__ __forceinline__ uint64_t selection_key(float act, uint32_t tie) {
@@ -1530,49 +1526,95 @@ __device__ __forceinline__ float surrogate_value(const LeoConfig& cfg, bool refr
 }
 
 // Phase-2 window of one wave in dynamic LDS (window_bytes per wave): the
-// touched neurons of a group of blocks in neuron order, their selection keys,
-// and per group block its first list position, candidate count and the key of
-// rank `limit`; plus the group's bitmap words and their list positions.
+// touched neurons of a run of blocks in any order, and those of them above
+// threshold (the candidates) with their selection keys and blocks. More than
+// 64 candidates are also sorted by block (`order`, `first`).
 struct Window {
-    uint64_t* key;     // capacity: selection key, ~0 for a non-candidate
-    uint64_t* cut;     // kGroupBlocks
-    uint32_t* entry;   // capacity: (group block << 16) | offset in the block
-    uint32_t* start;   // kGroupBlocks + 1
-    uint32_t* cands;   // kGroupBlocks
-    uint32_t* woff;    // kGroupBlocks: first staged winner position of each group block
-    uint32_t* bits;    // kWaveSize * kWordsPerLane: bitmap words of the group
-    uint32_t* pos;     // kWaveSize * kWordsPerLane: list position of each word's first bit
+    uint64_t* key;     // capacity: a candidate's selection key
+    uint32_t* entry;   // capacity: a touched neuron
+    uint32_t* block;   // capacity: a candidate's block, counted from the group's first
+    uint32_t* order;   // capacity: candidates by block
+    uint32_t* first;   // kGroupBlocks + 1: each block's first place in `order`
 };
 
 static_assert(kGroupBlocks == kWaveSize, "one lane per group block");
-static_assert(kMaxBlockNeurons <= 0x10000u, "window entries hold a 16-bit offset in the block");
 
 __device__ __forceinline__ Window wave_window(uint32_t wave, uint32_t nb) {
     unsigned char* base = step_lds + static_cast<size_t>(wave) * wave_lds_bytes(nb);
     const uint32_t cap = window_capacity(nb);
     Window w;
     w.key = reinterpret_cast<uint64_t*>(base);
-    w.cut = w.key + cap;
-    w.entry = reinterpret_cast<uint32_t*>(w.cut + kGroupBlocks);
-    w.start = w.entry + cap;
-    w.cands = w.start + kGroupBlocks + 1;
-    w.woff = w.cands + kGroupBlocks;
-    w.bits = w.woff + kGroupBlocks;
-    w.pos = w.bits + kWaveSize * kWordsPerLane;
+    w.entry = reinterpret_cast<uint32_t*>(w.key + cap);
+    w.block = w.entry + cap;
+    w.order = w.block + cap;
+    w.first = w.order + cap;
     return w;
+}
+
+// A candidate's rank in its block and its winner position: the candidates of
+// its block with smaller keys, and the winners of the blocks before its own
+// (of the window's `nc` candidates). A block's first `limit` candidates win.
+struct Placed {
+    uint32_t rank, before;
+};
+
+// Up to 64 candidates, one a lane: every pair through lane reads (a sparse
+// tick leaves a wave a few candidates). Every lane of the wave calls.
+__device__ __forceinline__ Placed place_few(uint64_t key, uint32_t block, uint32_t nc, uint32_t limit) {
+    Placed p{0, 0};
+    for (uint32_t q = 0; q < nc; ++q) {
+        const uint64_t kq = readlane_u64(key, q);
+        const uint32_t bq = __builtin_amdgcn_readlane(block, static_cast<int>(q));
+        p.rank += bq == block && kq < key ? 1u : 0u;
+    }
+    uint64_t winners = __ballot(__lane_id() < nc && p.rank < limit);
+    while (winners) {
+        const uint32_t q = static_cast<uint32_t>(__ffsll(static_cast<long long>(winners)) - 1);
+        winners &= winners - 1;
+        p.before += __builtin_amdgcn_readlane(block, static_cast<int>(q)) < block ? 1u : 0u;
+    }
+    return p;
+}
+
+// More than 64 candidates: sorted by block first (counts, a scan, places), so
+// that each is compared with its own block's candidates only. Leaves the
+// blocks' winner positions in `base` lanes (lane g: block g of the group).
+__device__ __forceinline__ uint32_t sort_by_block(const Window& w, uint32_t nc, uint32_t limit) {
+    const uint32_t lane = __lane_id();
+    w.first[lane] = 0u;
+    wave_sync();
+    for (uint32_t i = lane; i < nc; i += kWaveSize) atomicAdd(&w.first[w.block[i]], 1u);
+    wave_sync();
+    const uint32_t count = w.first[lane], won = min(count, limit);
+    const uint32_t start = wave_incl_scan_u32(count) - count;
+    wave_sync();
+    w.first[lane] = start;
+    wave_sync();
+    for (uint32_t i = lane; i < nc; i += kWaveSize) w.order[atomicAdd(&w.first[w.block[i]], 1u)] = i;
+    wave_sync();
+    w.first[lane] = start;
+    if (lane == 0) w.first[kGroupBlocks] = nc;
+    wave_sync();
+    return wave_incl_scan_u32(won) - won;
 }
 
 // Phase 2: each wave owns a range of blocks and takes it in groups of up to
 // kGroupBlocks blocks. Per group it loads (and clears) the group's touched
-// bitmap in one round of coalesced loads, lists the touched neurons in neuron
-// order, folds and drives them one lane each, and ranks every candidate within
-// its block: a candidate's rank is the number of smaller (activation desc, tie
-// asc) keys of its block, i.e. its position in the reference's sorted order
-// (runtime.rs:987-1011; keys are unique); rank `limit` gives the block cutoff.
-// The winners of the wave's range are staged in block order (runtime.rs:
-// 1010-1013), compacted from the range's first block row, so that phase 3
-// reads them in one round. A group with more touched neurons than the window
-// holds is taken in windows of whole blocks.
+// bitmap in one round of coalesced loads, lists the touched neurons (in the
+// words' lane order: one scan for the whole group), folds and drives them one
+// lane each, and places every candidate: its rank within its block is the
+// number of smaller (activation desc, tie asc) keys there, i.e. its position
+// in the reference's sorted order (runtime.rs:987-1011; keys are unique);
+// rank `limit` gives the block cutoff. The winners of the wave's range are
+// staged in block order (runtime.rs:1010-1013), compacted from the range's
+// first block row, so that phase 3 reads them in one round. A group with more
+// touched neurons than the window holds is taken in runs of whole blocks.
+// Bound by the chain of dependent instructions and memory rounds of one wave
+// per SIMD, not by bandwidth. Listing in neuron order took a scan and LDS
+// writes per row of 64 words, and block starts, counts and ranks went through
+// LDS: 470 frozen and 32 learning steps at a million units (33 blocks, ~22
+// touched neurons a wave) took 7.46 ms then and 7.07 now, a batch at 1,024
+// units (one block, ~84 touched neurons a wave) 74 ms then and 62 now.
 // `keep_bits`: a trace step leaves the bitmap words set for its eligibility
 // update (the learning phase clears them from the touched list). `pi` is the
 // population inhibition the previous tick left; `post_pending` that the
@@ -1597,192 +1639,163 @@ __device__ __forceinline__ void phase_fold_select(const StepCtx& c, StepShared& 
     const uint32_t set = set_of(d, tick);
     const FastDiv block_div = a.div_block_words;
     const Window w = wave_window(wave, nb);
-    w.cands[lane] = 0;
-    w.cut[lane] = ~0ULL;
+    uint32_t* deep_stage = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(w.key) + wave_window_bytes(nb));
     const uint64_t row0 = static_cast<uint64_t>(b0) * limit;
     // this wave's touched neurons are listed from its range's first neuron on
     // (no shared counter to wait for)
-    const uint32_t first_listed = b0 * nb;
-    uint32_t supra = 0, staged = 0, listed_before = 0, entries = 0;
+    uint32_t listed = b0 * nb;
+    uint32_t supra = 0, staged = 0, entries = 0;
+    // a candidate's place among the winners: staged for phase 3, or the cutoff
+    auto place = [&](uint64_t key, uint32_t block, const Placed& p) {
+        const float act = key_activation(key);
+        if (p.rank < limit) {
+            const uint32_t n = add_mod(static_cast<uint32_t>(key), rot, N);
+            const uint32_t k = staged + p.before + p.rank;  // staged position in the wave's range
+            const uint64_t at = row0 + k;
+            d.range_winners[at] = n;
+            d.range_winner_act[at] = act;
+            if (k < kWaveSize) {  // kept for phase 3 in the wave's LDS
+                sh.win_n[wave][k] = n;
+                sh.win_act[wave][k] = act;
+            }
+            if (a.redundant_global) {  // the global cap cannot bind (runtime.rs:1060-1067)
+                (*nf(d, n, kNActivation)) = act;
+                (*nu(d, n, kNSelected)) = tick + 1;
+            }
+        } else if (p.rank == limit && keep_bits) {
+            // read only by a trace step's eligibility update, as this tick's
+            // (by epoch): a block with no more candidates than winners keeps
+            // a stale epoch (cutoff 0)
+            d.block_cutoff[block] = act;
+            d.block_epoch[block] = tick + 1;
+        }
+    };
     for (uint32_t gb = b0; gb < b1; gb += group) {
         const uint32_t gn = min(group, b1 - gb), gw = gn * wpb;
-        uint32_t* bits = set_touched(d, set) + static_cast<uint64_t>(gb) * wpb;
-        uint32_t word[kWordsPerLane];
+        // the group's bitmap words through a buffer of exactly those words:
+        // loads past them return 0, so that no lane is masked
+        const __amdgpu_buffer_rsrc_t bits =
+            coherent_rsrc(set_touched(d, set) + static_cast<uint64_t>(gb) * wpb, gw * 4);
+        for (uint32_t s = 0; s < gn;) {
+            // the run of blocks [s, e): the rest of the group, or as many of
+            // its blocks as the window is sure to hold (a block holds at most
+            // nb <= cap); the words are loaded again for each run rather than
+            // kept in registers through the folds (a sparse tick has one run)
+            uint32_t word[kWordsPerLane];
 #pragma unroll
-        for (uint32_t k = 0; k < kWordsPerLane; ++k) {
-            const uint32_t at = k * kWaveSize + lane;
-            word[k] = at < gw ? ld(&bits[at]) : 0u;
-        }
-        // list positions in word order (row k holds words k*64 .. k*64+63);
-        // each row's neurons are listed as soon as its positions are known
-        // (the words are in registers), at positions below the window
-        // capacity: a group that fits the window is then fully listed
-        uint32_t total = 0;
+            for (uint32_t k = 0; k < kWordsPerLane; ++k) {
+                word[k] = 0u;
+                if (k * kWaveSize < gw)
+                    word[k] = __builtin_amdgcn_raw_buffer_load_b32(bits, (k * kWaveSize + lane) * 4, 0, 16);
+            }
+            if (s > 0) {
 #pragma unroll
-        for (uint32_t k = 0; k < kWordsPerLane; ++k) {
-            const uint32_t at = k * kWaveSize + lane;
-            if (k * kWaveSize < gw) {
-                const uint32_t cnt = __popc(word[k]);
-                const uint32_t incl = wave_incl_scan_u32(cnt);
-                uint32_t p = total + incl - cnt;
-                w.bits[at] = word[k];
-                w.pos[at] = p;
+                for (uint32_t k = 0; k < kWordsPerLane; ++k)
+                    if (k * kWaveSize + lane < s * wpb) word[k] = 0u;
+            }
+            uint32_t e = gn, incl = 0, total = 0;
+            for (;;) {
+                uint32_t part = 0;
+#pragma unroll
+                for (uint32_t k = 0; k < kWordsPerLane; ++k) part += __popc(word[k]);
+                incl = wave_incl_scan_u32(part);
+                total = __builtin_amdgcn_readlane(incl, kWaveSize - 1);
+                if (__builtin_expect(total <= cap, 1) || e == s + 1) break;
+                e = s + (e - s + 1) / 2;
+#pragma unroll
+                for (uint32_t k = 0; k < kWordsPerLane; ++k)
+                    if (k * kWaveSize + lane >= e * wpb) word[k] = 0u;
+            }
+            // the words are cleared after all have arrived: a store issued
+            // between the loads would be waited for together with the later
+            // ones (clearing every word, set or not, was slower: 0.4 us of a
+            // frozen step at a million units)
+            if (!keep_bits) {
+#pragma unroll
+                for (uint32_t k = 0; k < kWordsPerLane; ++k) {
+                    if (word[k]) __builtin_amdgcn_raw_buffer_store_b32(0u, bits, (k * kWaveSize + lane) * 4, 0, 0);
+                }
+            }
+            uint32_t p = incl;  // this lane's neurons end here
+#pragma unroll
+            for (uint32_t k = 0; k < kWordsPerLane; ++k) {
                 uint32_t v = word[k];
-                if (v != 0 && p < cap) {
-                    const uint32_t g = fast_div(at, block_div), base = (at - g * wpb) * 32;
-                    while (v) {
-                        const uint32_t bit = __ffs(v) - 1;
+                if (k * kWaveSize < gw && v != 0) {
+                    const uint32_t at = k * kWaveSize + lane, g = fast_div(at, block_div);
+                    const uint32_t n0 = (gb + g) * nb + (at - g * wpb) * 32;
+                    do {
+                        w.entry[--p] = n0 + __ffs(v) - 1;
                         v &= v - 1;
-                        if (p < cap) w.entry[p] = (g << 16) | (base + bit);
-                        ++p;
-                    }
-                }
-                total += __builtin_amdgcn_readlane(incl, kWaveSize - 1);
-            }
-        }
-        // the words are cleared after the scan: a store issued between the
-        // rows would be waited for together with the next row's words
-#pragma unroll
-        for (uint32_t k = 0; k < kWordsPerLane; ++k) {
-            const uint32_t at = k * kWaveSize + lane;
-            if (!keep_bits && at < gw && word[k]) bits[at] = 0u;
-        }
-        // block starts: the list position of each block's first word
-        wave_sync();
-        if (lane < gn) w.start[lane] = w.pos[lane * wpb];
-        if (lane == 0) w.start[gn] = total;
-        wave_sync();
-        for (uint32_t lo = 0; lo < total;) {
-            uint32_t hi = total;
-            if (total - lo > cap) {
-                // the last block boundary within the window (a block holds at most nb <= cap)
-                uint32_t best = lo;
-                for (uint32_t g = lane; g <= gn; g += kWaveSize) {
-                    const uint32_t st = w.start[g];
-                    if (st <= lo + cap && st > best) best = st;
-                }
-                hi = static_cast<uint32_t>(wave_max_u64(best));
-            }
-            for (uint32_t k = 0; total > cap && k < kWordsPerLane; ++k) {  // else listed in the scan
-                const uint32_t at = k * kWaveSize + lane;
-                if (at >= gw) break;
-                uint32_t v = w.bits[at], p = w.pos[at];
-                if (p >= hi || p + __popc(v) <= lo) continue;
-                const uint32_t g = fast_div(at, block_div), base = (at - g * wpb) * 32;
-                while (v) {
-                    const uint32_t bit = __ffs(v) - 1;
-                    v &= v - 1;
-                    if (p >= lo && p < hi) w.entry[p - lo] = (g << 16) | (base + bit);
-                    ++p;
+                    } while (v);
                 }
             }
             wave_sync();
-            const uint32_t cnt = hi - lo;
-            const uint32_t listed = first_listed + listed_before + lo;
-            bool any_deep = false;
-            for (uint32_t i = lane; i < cnt; i += kWaveSize) {
-                const uint32_t e = w.entry[i];
-                const uint32_t g = e >> 16;
-                const uint32_t n = (gb + g) * nb + (e & 0xffffu);
+            uint32_t nc = 0;
+            for (uint32_t i0 = 0; i0 < total; i0 += kWaveSize) {
+                const bool valid = i0 + lane < total;
                 bool refractory = false, deep = false;
-                uint32_t folded = 0;
-                const float act = clampf(fold_drive(c, n, pi, set, post_pending, &refractory, &deep, &folded), 0.0f, 1.0f);
+                uint32_t folded = 0, n = 0;
+                float act = 0.0f;
+                if (valid) {
+                    n = w.entry[i0 + lane];
+                    act = clampf(fold_drive(c, n, pi, set, post_pending, &refractory, &deep, &folded), 0.0f, 1.0f);
+                    if (keep_bits) d.touched_list[listed + i0 + lane] = n;  // read by a trace step's homeostasis only
+                }
                 entries += folded;
-                const bool candidate = !deep && !refractory && act > 0.0f;
-                w.key[i] = deep ? kDeepPending : candidate ? selection_key(act, add_mod(n, N - rot, N)) : ~0ULL;
-                any_deep |= deep;
-                if (candidate) atomicAdd(&w.cands[g], 1u);
-                if (keep_bits) d.touched_list[listed + i] = n;  // read by a trace step's homeostasis only
-            }
-            wave_sync();
-            if (__ballot(any_deep)) {
+                const bool candidate = valid && !deep && !refractory && act > 0.0f;
+                const uint64_t found = __ballot(candidate);
+                if (candidate) {
+                    const uint32_t at = nc + static_cast<uint32_t>(__popcll(found & ((1ULL << lane) - 1ULL)));
+                    w.key[at] = selection_key(act, add_mod(n, N - rot, N));
+                    w.block[at] = fast_div(n, a.div_block) - gb;
+                }
+                nc += static_cast<uint32_t>(__popcll(found));
                 // neurons with more than 8 deliveries: the whole wave folds each
-                uint32_t* hist = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(w.key) +
-                                                             wave_window_bytes(nb));
-                for (uint32_t i0 = 0; i0 < cnt; i0 += kWaveSize) {
-                    uint64_t pending = __ballot(i0 + lane < cnt && w.key[i0 + lane] == kDeepPending);
-                    while (pending) {
-                        const uint32_t i = i0 + static_cast<uint32_t>(__ffsll(static_cast<long long>(pending)) - 1);
-                        pending &= pending - 1;
-                        const uint32_t e = __builtin_amdgcn_readfirstlane(w.entry[i]);
-                        const uint32_t g = e >> 16;
-                        const uint32_t n = (gb + g) * nb + (e & 0xffffu);
-                        bool refractory = false;
-                        const float act = clampf(deep_fold(c, n, pi, set, post_pending, &refractory, hist), 0.0f, 1.0f);
-                        const bool candidate = !refractory && act > 0.0f;
+                uint64_t pending = __ballot(deep);
+                while (pending) {
+                    const uint32_t q = static_cast<uint32_t>(__ffsll(static_cast<long long>(pending)) - 1);
+                    pending &= pending - 1;
+                    const uint32_t dn = __builtin_amdgcn_readlane(n, static_cast<int>(q));
+                    bool refr = false;
+                    const float dact = clampf(deep_fold(c, dn, pi, set, post_pending, &refr, deep_stage), 0.0f, 1.0f);
+                    if (!refr && dact > 0.0f) {
                         if (lane == 0) {
-                            w.key[i] = candidate ? selection_key(act, add_mod(n, N - rot, N)) : ~0ULL;
-                            if (candidate) atomicAdd(&w.cands[g], 1u);
+                            w.key[nc] = selection_key(dact, add_mod(dn, N - rot, N));
+                            w.block[nc] = fast_div(dn, a.div_block) - gb;
                         }
-                        wave_sync();
+                        nc += 1;
                     }
-                }
-            }
-            {
-                // staged positions of this window's blocks (block order)
-                const bool in = lane < gn && w.start[lane] >= lo && w.start[lane] < hi;
-                const uint32_t win = in ? min(w.cands[lane], limit) : 0u;
-                const uint32_t incl = wave_incl_scan_u32(win);
-                if (in) w.woff[lane] = staged + incl - win;
-                staged += __builtin_amdgcn_readlane(incl, kWaveSize - 1);
-            }
-            wave_sync();
-            for (uint32_t i = lane; i < cnt; i += kWaveSize) {
-                const uint64_t mine = w.key[i];
-                if (mine == ~0ULL) continue;
-                const uint32_t g = w.entry[i] >> 16;
-                const uint32_t s0 = w.start[g] - lo, s1 = w.start[g + 1] - lo;
-                uint32_t rank = 0;
-                // eight independent LDS reads in flight per round (one read
-                // at a time waits out the LDS latency on every key)
-                uint32_t j = s0;
-                for (; j + 8 <= s1; j += 8) {
-                    uint64_t k[8];
-#pragma unroll
-                    for (uint32_t x = 0; x < 8; ++x) k[x] = w.key[j + x];
-#pragma unroll
-                    for (uint32_t x = 0; x < 8; ++x) rank += k[x] < mine ? 1u : 0u;
-                }
-                for (; j < s1; ++j) rank += w.key[j] < mine ? 1u : 0u;
-                if (rank < limit) {
-                    const uint32_t n = add_mod(static_cast<uint32_t>(mine), rot, N);
-                    const float act = key_activation(mine);
-                    const uint32_t k = w.woff[g] + rank;  // staged position in the wave's range
-                    const uint64_t at = row0 + k;
-                    d.range_winners[at] = n;
-                    d.range_winner_act[at] = act;
-                    if (k < kWaveSize) {  // kept for phase 3 in the wave's LDS
-                        sh.win_n[wave][k] = n;
-                        sh.win_act[wave][k] = act;
-                    }
-                    if (a.redundant_global) {  // the global cap cannot bind (runtime.rs:1060-1067)
-                        (*nf(d, n, kNActivation)) = act;
-                        (*nu(d, n, kNSelected)) = tick + 1;
-                    }
-                } else if (rank == limit) {
-                    w.cut[g] = mine;
                 }
             }
             wave_sync();
-            lo = hi;
-        }
-        // block results, read only by a trace step's eligibility update (as
-        // this tick's, by epoch); a block without touched neurons keeps a
-        // stale epoch (no winners, cutoff 0)
-        if (lane < gn && w.start[lane + 1] > w.start[lane]) {
-            const uint32_t b = gb + lane;
-            if (keep_bits) {
-                d.block_cutoff[b] = w.cut[lane] != ~0ULL ? key_activation(w.cut[lane]) : 0.0f;
-                d.block_epoch[b] = tick + 1;
+            if (nc <= kWaveSize) {
+                const uint64_t key = lane < nc ? w.key[lane] : ~0ULL;
+                const uint32_t block = lane < nc ? w.block[lane] : ~0u;
+                const Placed at = place_few(key, block, nc, limit);
+                if (lane < nc) place(key, gb + block, at);
+                staged += static_cast<uint32_t>(__popcll(__ballot(lane < nc && at.rank < limit)));
+            } else {
+                const uint32_t base = sort_by_block(w, nc, limit);
+                uint32_t won = 0;
+                for (uint32_t i0 = 0; i0 < nc; i0 += kWaveSize) {
+                    const uint32_t i = i0 + lane;
+                    const uint64_t key = i < nc ? w.key[i] : ~0ULL;
+                    const uint32_t block = i < nc ? w.block[i] : 0u;
+                    Placed at{0, static_cast<uint32_t>(__shfl(static_cast<int>(base), static_cast<int>(block)))};
+                    const uint32_t j1 = i < nc ? w.first[block + 1] : 0u;
+                    for (uint32_t j = w.first[block]; j < j1; ++j) at.rank += w.key[w.order[j]] < key ? 1u : 0u;
+                    if (i < nc) place(key, gb + block, at);
+                    won += static_cast<uint32_t>(__popcll(__ballot(i < nc && at.rank < limit)));
+                }
+                staged += won;
             }
-            supra += w.cands[lane];
+            wave_sync();
+            supra += nc;
+            listed += total;
+            s = e;
         }
-        w.cands[lane] = 0;
-        w.cut[lane] = ~0ULL;
-        listed_before += total;
-        wave_sync();
     }
-    supra = wave_sum_u32(supra);
+    const uint32_t listed_before = listed - b0 * nb;
     entries = wave_sum_u32(entries);
     if (lane == 0) {
         if (c.tally) {
@@ -3662,13 +3675,15 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
 
 // The arguments live in device memory (read with scalar loads): a by-value
 // argument whose address is taken is copied to scratch.
-__global__ void __launch_bounds__(kThreads) leo_lane_steps(const KernelArgs* __restrict__ args) {
+// Two waves per SIMD at the least: the cooperative capacity is planned for two
+// workgroups per CU, so the compiler keeps within 256 registers.
+__global__ void __launch_bounds__(kThreads, 2) leo_lane_steps(const KernelArgs* __restrict__ args) {
     lane_steps<false, false>(*args);
 }
-__global__ void __launch_bounds__(kThreads) leo_lane_steps_profiled(const KernelArgs* __restrict__ args) {
+__global__ void __launch_bounds__(kThreads, 2) leo_lane_steps_profiled(const KernelArgs* __restrict__ args) {
     lane_steps<true, false>(*args);
 }
-__global__ void __launch_bounds__(kThreads) leo_lane_steps_frozen(const KernelArgs* __restrict__ args) {
+__global__ void __launch_bounds__(kThreads, 2) leo_lane_steps_frozen(const KernelArgs* __restrict__ args) {
     lane_steps<false, true>(*args);
 }
 
