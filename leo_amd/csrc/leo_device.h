@@ -33,6 +33,7 @@ constexpr uint32_t kEndIndex = 256;
 constexpr uint32_t kRing = 9;             // delay ring: max delay 8 + 1 (runtime.rs:200-208)
 constexpr uint32_t kBucketSets = kRing;   // delivery bucket sets of a lane with one-barrier frozen runs
 constexpr uint32_t kMaxOrder = 16;        // config.rs:452-456
+constexpr uint32_t kMaxEmbedding = 256;   // config.rs:447-451
 constexpr uint32_t kThreads = 256;        // threads per workgroup
 constexpr uint32_t kMaxBlockNeurons = 1024;
 constexpr uint32_t kWaveSize = 64;

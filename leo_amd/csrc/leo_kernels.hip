@@ -185,19 +185,30 @@ __device__ __forceinline__ uint32_t wave_incl_scan_u32(uint32_t v) {
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
     return __builtin_amdgcn_readlane(wave_incl_scan_u32(v), kWaveSize - 1);
 }
-__device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long v) {
-    for (int off = 32; off > 0; off >>= 1) {
-        unsigned long long o = __shfl_xor(v, off);
-        v = o < v ? o : v;
-    }
-    return v;
+// Maxima over the wave (every lane must be active), uniform; lanes without a
+// source keep their own value. The float maximum ignores NaNs like maxnum.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ uint32_t dpp_keep_u32(uint32_t x) {
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(static_cast<int>(x), static_cast<int>(x), kCtrl, kRowMask, 0xf, false));
 }
-__device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {
-    for (int off = 32; off > 0; off >>= 1) {
-        unsigned long long o = __shfl_xor(v, off);
-        v = o > v ? o : v;
-    }
-    return v;
+template <class Max>
+__device__ __forceinline__ uint32_t wave_reduce_max(uint32_t v, Max&& larger) {
+    v = larger(v, dpp_keep_u32<0x111, 0xf>(v));
+    v = larger(v, dpp_keep_u32<0x112, 0xf>(v));
+    v = larger(v, dpp_keep_u32<0x114, 0xf>(v));
+    v = larger(v, dpp_keep_u32<0x118, 0xf>(v));
+    v = larger(v, dpp_keep_u32<0x142, 0xa>(v));
+    v = larger(v, dpp_keep_u32<0x143, 0xc>(v));
+    return __builtin_amdgcn_readlane(v, kWaveSize - 1);
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    return wave_reduce_max(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+}
+__device__ __forceinline__ float wave_max_f32(float v) {
+    return __uint_as_float(wave_reduce_max(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(maxnum(__uint_as_float(a), __uint_as_float(b)));
+    }));
 }
 // Index of the calling wave in its workgroup, known to the compiler as uniform
 // (values derived from it live in scalar registers).
@@ -449,14 +460,21 @@ struct alignas(16) StepShared {
     float err[kOutStride];                                      // errors / logits
     float aux[kOutStride + kThreads];                           // exps, latent, gradient
     uint32_t scan[kThreads];
-    unsigned long long red[kWavesPerGroup];
-    float redf[kWavesPerGroup];
+    uint32_t red[3][kWavesPerGroup];
+    float redf[2][kWavesPerGroup];
     // context resolution (one thread per order)
     uint32_t hist[kMaxOrder];
     int64_t ctx_slot[kMaxOrder];
     float ctx_scale[kMaxOrder];
     uint32_t ctx_probes[kMaxOrder];
     uint32_t hist_len;
+    // the resolved context's cells and scales, its latent and its contribution
+    // to the logits (context_logits)
+    uint32_t ctx_cells;
+    uint32_t ctx_cell[kMaxOrder];
+    float ctx_weight[kMaxOrder];
+    float latent[kMaxEmbedding];
+    float ctx_logit[kOutStride];
     // this workgroup's copy of the emission ring bookkeeping (LaneControl ring_*)
     uint32_t ring_tick[kRing];
     uint32_t ring_count[kRing];
@@ -1027,13 +1045,18 @@ __device__ __forceinline__ void context_resolve(const StepCtx& c, const StepPara
                 probes += sh.ctx_probes[t];
                 if (sh.ctx_slot[t] < 0) continue;
                 ctl->ctx_slots[count] = static_cast<uint32_t>(sh.ctx_slot[t]);
+                sh.ctx_cell[count] = static_cast<uint32_t>(sh.ctx_slot[t]);
                 scales[count] = sh.ctx_scale[t];
                 scale_sum += sh.ctx_scale[t];
                 count += 1;
             }
-            for (uint32_t i = 0; i < count; ++i)
-                ctl->ctx_scales[i] = scale_sum > 0.0f ? scales[i] / scale_sum : scales[i];
+            for (uint32_t i = 0; i < count; ++i) {
+                const float scale = scale_sum > 0.0f ? scales[i] / scale_sum : scales[i];
+                ctl->ctx_scales[i] = scale;
+                sh.ctx_weight[i] = scale;
+            }
         }
+        sh.ctx_cells = count;
         ctl->ctx_applied = enabled ? 1u : 0u;
         ctl->ctx_count = count;
         ctl->ctx_probes = probes;
@@ -1843,8 +1866,11 @@ __device__ __forceinline__ void write_active(const StepCtx& c, const StepParams&
     // first memory round: the per-wave totals, this wave's winners' state and first
     // synapses, and this thread's first item of the next tick
     // the recording wave's loads go out in the same round; it runs on the
-    // workgroup that selects nothing (the least work in this phase)
-    const bool rec_wave = c.part == c.P - 1 && wave == 0;
+    // workgroup that selects nothing, except on a frozen step with a readout,
+    // which that workgroup alone works on (the record took 2.4 us in front
+    // of it)
+    const bool readout_only = (sp.flags & kStepOutput) && !(sp.flags & kStepLearnTrace);
+    const bool rec_wave = c.part == (readout_only ? 0 : c.P - 1) && wave == 0;
     const bool recorder = rec_wave && lane == 0;
     float pi_old = 0.0f;
     uint32_t supra = 0, rec_n = 0, in_n = 0, cells = 0, probes = 0, applied = 0;
@@ -2681,19 +2707,39 @@ __device__ __forceinline__ void phase_eligibility(const StepCtx& c, bool plastic
 }
 
 // The serial sum of kOutputs values in LDS (runtime.rs:1175-1180 order),
-// read sixteen at a time in 16-byte loads (one read at a time would wait out
-// the LDS latency on every term).
+// read sixteen at a time in 16-byte loads, the next sixteen while the current
+// ones are added (one read at a time would wait out the LDS latency on every
+// term; unrolled further, the reads of every group would be hoisted into 256
+// registers).
 __device__ __forceinline__ float serial_sum_outputs(const float* v) {
     static_assert(kOutputs == 257, "256 values in sixteen-value groups, then the last");
     const f32x4* v4 = reinterpret_cast<const f32x4*>(v);
     float sum = 0.0f;
-    for (uint32_t g = 0; g < 64; g += 4) {
-        const f32x4 a = v4[g], b = v4[g + 1], c = v4[g + 2], e = v4[g + 3];
-        sum += a.x; sum += a.y; sum += a.z; sum += a.w;
-        sum += b.x; sum += b.y; sum += b.z; sum += b.w;
-        sum += c.x; sum += c.y; sum += c.z; sum += c.w;
-        sum += e.x; sum += e.y; sum += e.z; sum += e.w;
+    f32x4 a[4], b[4];
+    auto load = [&](f32x4(&x)[4], uint32_t g) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) x[k] = v4[g + k];
+    };
+    auto add = [&](const f32x4(&x)[4]) {
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            sum += x[k].x;
+            sum += x[k].y;
+            sum += x[k].z;
+            sum += x[k].w;
+        }
+    };
+    load(a, 0);
+#pragma unroll 1
+    for (uint32_t g = 0; g < 56; g += 8) {
+        load(b, g + 4);
+        add(a);
+        load(a, g + 8);
+        add(b);
     }
+    load(b, 60);
+    add(a);
+    add(b);
     return sum + v[256];
 }
 
@@ -2702,251 +2748,269 @@ __device__ __forceinline__ float serial_sum_outputs(const float* v) {
 // (runtime.rs:1084-1106), and on the last workgroup the readout, softmax and
 // errors (runtime.rs:1108-1197, 1205-1206).
 // ---------------------------------------------------------------------------
+// The context's share of an output step's logits (runtime.rs:1120-1149), by
+// the last workgroup in phase 2, where it selects no blocks: neither the cells
+// nor the projection change before the learning phase, so the readout, which
+// ends phase 3, finds the sums in LDS. The latent is serial over the cells per
+// dimension, a logit's contribution serial over the dimensions.
+__device__ __forceinline__ void context_logits(const StepCtx& c, StepShared& sh) {
+    const LaneDesc& d = c.d;
+    const uint32_t E = c.a->cfg.context_embedding_dim;
+    const uint32_t cells = __builtin_amdgcn_readfirstlane(sh.ctx_cells);
+    for (uint32_t e = threadIdx.x; e < E; e += kThreads) {
+        float emb[kMaxOrder];
+#pragma unroll
+        for (uint32_t i = 0; i < kMaxOrder; ++i)
+            emb[i] = i < cells ? ld(&d.p.ctx_emb[static_cast<uint64_t>(sh.ctx_cell[i]) * E + e]) : 0.0f;
+        float v = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < kMaxOrder; ++i)
+            if (i < cells && sh.ctx_weight[i] > 0.0f) v += emb[i] * sh.ctx_weight[i];
+        sh.latent[e] = v;
+        d.ctx_latent[e] = v;
+    }
+    if (cells == 0) return;
+    __syncthreads();
+    const __amdgpu_buffer_rsrc_t proj = coherent_rsrc(d.p.ctx_out, kOutputs * E * 4);
+    for (uint32_t o = threadIdx.x; o < kOutputs; o += kThreads) {
+        float v = 0.0f;
+        uint32_t e = 0;
+        if ((E & 3u) == 0) {  // rows of whole 16-byte quarters
+            for (; e + 16 <= E; e += 16) {
+                f32x4 x[4];
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) x[k] = ld16(proj, (o * E + e + 4 * k) * 4);
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    v += x[k].x * sh.latent[e + 4 * k];
+                    v += x[k].y * sh.latent[e + 4 * k + 1];
+                    v += x[k].z * sh.latent[e + 4 * k + 2];
+                    v += x[k].w * sh.latent[e + 4 * k + 3];
+                }
+            }
+        }
+        for (; e < E; ++e) v += ld4(proj, (o * E + e) * 4) * sh.latent[e];
+        sh.ctx_logit[o] = v;
+    }
+}
+
+// The readout's list of active neurons, from the selecting waves' winners (the
+// active list of a non-binding cap, still being written in this phase): the
+// ids and activations of list places [b0, b0 + kThreads) into LDS, one thread
+// per selecting wave, its first winner loaded with its total. Returns the
+// list's length.
+__device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& sh, uint32_t b0, uint32_t* ids, float* acts) {
+    const LaneDesc& d = c.d;
+    const LeoConfig& cfg = c.a->cfg;
+    const uint32_t nwaves = selecting_waves(c), wave = wave_index(), lane = __lane_id();
+    const uint32_t range = (cfg.block_count + nwaves - 1) / nwaves;
+    uint32_t running = 0;
+    for (uint32_t base = 0; base < nwaves; base += kThreads) {
+        const uint32_t wv = base + threadIdx.x;
+        const bool owns = wv < nwaves && wv * range < cfg.block_count;
+        const uint64_t row0 = static_cast<uint64_t>(wv) * range * cfg.max_active_per_block;
+        const uint32_t count = owns ? ld(&wave_totals(d, c.tick)[wv]) : 0u;
+        const uint32_t n0 = owns ? ld(&d.range_winners[row0]) : 0u;
+        const float act0 = owns ? ld(&d.range_winner_act[row0]) : 0.0f;
+        const uint32_t incl = wave_incl_scan_u32(count);
+        if (lane == kWaveSize - 1) sh.red[0][wave] = incl;
+        __syncthreads();
+        uint32_t at = running + incl - count;
+#pragma unroll
+        for (uint32_t w = 0; w < kWavesPerGroup; ++w) {
+            const uint32_t total = sh.red[0][w];
+            at += w < wave ? total : 0u;
+            running += total;
+        }
+        for (uint32_t i = 0; i < count; ++i) {
+            const uint32_t f = at + i - b0;  // wraps past kThreads below b0
+            if (f >= kThreads) continue;
+            ids[f] = i == 0 ? n0 : ld(&d.range_winners[row0 + i]);
+            acts[f] = i == 0 ? act0 : ld(&d.range_winner_act[row0 + i]);
+        }
+        __syncthreads();
+    }
+    return running;
+}
+
 // The readout runs in phase 3, beside the eligibility update, on the last
 // workgroup (which selects no blocks); the post phase leaves its record
 // fields alone. With a non-binding global cap the active list is still being
 // written in that phase, so the readout takes it from the selecting waves'
 // winners (block order: the same list); otherwise the global selection has
 // written it before the phase's first barrier.
+// One workgroup's chain of dependent rounds: (1) the winners with the bias,
+// (2) the rows of 32 active neurons at a time (thread t owns output t; the
+// end-class weights are gathered one neuron a thread and added by thread 0),
+// then the softmax: maxima through DPP, every wave sums the exponentials
+// itself (serial, so no broadcast), and one exchange for the argmax and the
+// bias check. An evaluated step at 16,384 units spent 11.8 us in this phase
+// with the context loads in it, an LDS scan of the winner totals, a search per
+// winner and shuffled reductions; 7.0 us now (winners 0.8, rows 1.5, maxima
+// 0.7, exponentials 0.8, sum 0.7, the rest 1.2).
 __device__ __forceinline__ void readout(const StepCtx& c, const StepParams& sp, StepShared& sh, uint32_t step_index) {
     const KernelArgs& a = *c.a;
     const LaneDesc& d = c.d;
     const LeoConfig& cfg = a.cfg;
     LaneControl* ctl = c.ctl;
-    const uint32_t cap = cfg.max_active_global, E = cfg.context_embedding_dim;
     const uint32_t rs = c.tick % kRing;
-    const uint32_t* act_list = d.ring_active + static_cast<uint64_t>(rs) * cap;
-    const float* act_val = d.ring_act + static_cast<uint64_t>(rs) * cap;
     const uint32_t wave = wave_index(), lane = __lane_id();
-    const uint32_t o1 = threadIdx.x, o2 = threadIdx.x + kThreads;
-    const bool has2 = o2 < kOutputs;
-    float* lat = sh.aux;
-    // Memory rounds: (1) the context count, slots and scales, the bias and
-    // the waves' winner totals; (2) the context embeddings; (3) the first 256
-    // active ids and activations (into LDS) with this thread's first 16
-    // context-projection weights; (4) rows of 32 active neurons at a time.
-    // (A load's wait also waits for every load issued before it, so the
-    // projection weights, needed last, go out after the embeddings.)
-    const bool from_waves = a.redundant_global != 0;
-    uint32_t* starts = reinterpret_cast<uint32_t*>(step_lds + 2 * kThreads * 4);
-    const uint32_t nwaves = selecting_waves(c);
-    const uint32_t range = (cfg.block_count + nwaves - 1) / nwaves;
-    const uint32_t N = cfg.neuron_count, rot = c.tick % N;
-    if (threadIdx.x == 0) {
-        d.records[step_index].p_target = 0.0f;
-        d.records[step_index].predicted = 0;
-    }
-    // the slots past the count are loaded too (and not used), so that the
-    // slots do not wait for the count
-    const uint32_t ctx_count = ld(&ctl->ctx_count);
-    uint32_t slot[kMaxOrder];
-    float scale[kMaxOrder];
-#pragma unroll
-    for (uint32_t i = 0; i < kMaxOrder; ++i) {
-        slot[i] = threadIdx.x < E ? ld(&ctl->ctx_slots[i]) : 0u;
-        scale[i] = threadIdx.x < E ? ld(&ctl->ctx_scales[i]) : 0.0f;
-    }
-    float l1 = ld(&d.p.bias[o1]), l2 = has2 ? ld(&d.p.bias[o2]) : 0.0f;
-    const float bias1 = l1, bias2 = l2;
-    const uint32_t A = from_waves ? wave_starts(c, sh, starts, nwaves) : ld(&ctl->active_count);
-    // context latent (runtime.rs:1120-1136): serial over active slots per
-    // dimension
-    for (uint32_t e = threadIdx.x; e < E; e += kThreads) {
-        float emb[kMaxOrder];
-#pragma unroll
-        for (uint32_t i = 0; i < kMaxOrder; ++i)
-            emb[i] = i < ctx_count && scale[i] > 0.0f ? ld(&d.p.ctx_emb[static_cast<uint64_t>(slot[i]) * E + e]) : 0.0f;
-        float v = 0.0f;
-#pragma unroll
-        for (uint32_t i = 0; i < kMaxOrder; ++i)
-            if (i < ctx_count && scale[i] > 0.0f) v += emb[i] * scale[i];
-        lat[e] = v;
-        d.ctx_latent[e] = v;
-    }
-    constexpr uint32_t kDims = 16;
-    float x1[kDims], x2[kDims];
-#pragma unroll
-    for (uint32_t k = 0; k < kDims; ++k) {
-        x1[k] = k < E ? ld(&d.p.ctx_out[o1 * E + k]) : 0.0f;
-        x2[k] = k < E && has2 ? ld(&d.p.ctx_out[o2 * E + k]) : 0.0f;
-    }
-    // logits[o] = bias[o] + sum over active in order of W[n][o]*a_n (+ context
-    // once): thread t owns outputs t and t+256; the active ids and
-    // activations are staged in LDS 256 at a time, then the rows of 32
-    // neurons go out together ahead of the serial adds
-    // (ids past the block's end read row 0 and are not added, so the row
-    // loads carry no conditions and go out back to back)
+    const uint32_t o1 = threadIdx.x;
+    const bool end_thread = threadIdx.x == 0;  // also owns the end class
     uint32_t* ids = reinterpret_cast<uint32_t*>(step_lds);
     float* acts = reinterpret_cast<float*>(step_lds) + kThreads;
+    float* ends = reinterpret_cast<float*>(step_lds) + 2 * kThreads;
+    StepRecord LEO_GLOBAL& rec = d.records[step_index];
+    if (end_thread) {
+        rec.p_target = 0.0f;
+        rec.predicted = 0;
+    }
+    const bool from_waves = a.redundant_global != 0;
+    float l1 = ld(&d.p.bias[o1]), l2 = end_thread ? ld(&d.p.bias[kEndIndex]) : 0.0f;
+    const float bias1 = l1, bias2 = l2;
+    uint32_t A = from_waves ? 0u : ld(&ctl->active_count);
+    // logits[o] = bias[o] + sum over active in order of W[n][o]*a_n (+ context
+    // once): the active ids and activations are staged in LDS 256 at a time,
+    // then the rows of 32 neurons go out together ahead of the serial adds
+    // (ids past the block's end read row 0 and are not added, so the row
+    // loads carry no conditions and go out back to back)
     constexpr uint32_t kRows = 32;
     static_assert(kThreads % kRows == 0, "whole row chunks per block of ids");
-    for (uint32_t b0 = 0; b0 < A; b0 += kThreads) {
-        const uint32_t bn = min(kThreads, A - b0);
-        __syncthreads();  // the previous block's ids are consumed (and the latent is written)
-        if (from_waves) {
-            uint32_t n = 0;
-            float act = 0.0f;
-            if (threadIdx.x < bn)
-                (void)winner_key(d, starts, nwaves, range, cfg.block_count, cfg.max_active_per_block,
-                                 b0 + threadIdx.x, N, rot, &n, &act);
-            ids[threadIdx.x] = n;
-            if (threadIdx.x < bn) acts[threadIdx.x] = act;
-        } else {
-            ids[threadIdx.x] = threadIdx.x < bn ? ld(&act_list[b0 + threadIdx.x]) : 0u;
-            if (threadIdx.x < bn) acts[threadIdx.x] = ld(&act_val[b0 + threadIdx.x]);
-        }
+    auto row_weight = [&](uint32_t n) {  // every lane holds the same id: a scalar row address
+        const float LEO_GLOBAL* row =
+            d.p.out_w + static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(n)) * kOutStride;
+        return ld(&row[o1]);
+    };
+    for (uint32_t b0 = 0; b0 == 0 || b0 < A; b0 += kThreads) {
+        ids[threadIdx.x] = 0u;
         __syncthreads();
+        if (from_waves) {
+            A = list_winners(c, sh, b0, ids, acts);
+        } else if (b0 + threadIdx.x < A) {
+            const uint64_t at = static_cast<uint64_t>(rs) * cfg.max_active_global + b0 + threadIdx.x;
+            ids[threadIdx.x] = ld(&d.ring_active[at]);
+            acts[threadIdx.x] = ld(&d.ring_act[at]);
+        }
+        if (!from_waves) __syncthreads();
+        const uint32_t bn = min(kThreads, A - b0);
+        if (threadIdx.x < bn)
+            ends[threadIdx.x] = ld(&d.p.out_w[static_cast<uint64_t>(ids[threadIdx.x]) * kOutStride + kEndIndex]) *
+                                acts[threadIdx.x];
         for (uint32_t r0 = 0; r0 < bn; r0 += kRows) {
-            float w1[kRows], w2[kRows];
-            uint32_t n[kRows];
+            float w1[kRows];
             const uint4* ids4 = reinterpret_cast<const uint4*>(ids + r0);
 #pragma unroll
             for (uint32_t k = 0; k < kRows / 4; ++k) {
                 const uint4 q = ids4[k];
-                n[4 * k] = q.x;
-                n[4 * k + 1] = q.y;
-                n[4 * k + 2] = q.z;
-                n[4 * k + 3] = q.w;
+                w1[4 * k] = row_weight(q.x);
+                w1[4 * k + 1] = row_weight(q.y);
+                w1[4 * k + 2] = row_weight(q.z);
+                w1[4 * k + 3] = row_weight(q.w);
             }
-#pragma unroll
-            for (uint32_t k = 0; k < kRows; ++k) {
-                const float* row = d.p.out_w + static_cast<uint64_t>(n[k]) * kOutStride;
-                w1[k] = ld(&row[o1]);
-                w2[k] = has2 ? ld(&row[o2]) : 0.0f;
-            }
-            float av[kRows];
             const f32x4* acts4 = reinterpret_cast<const f32x4*>(acts + r0);
 #pragma unroll
             for (uint32_t k = 0; k < kRows / 4; ++k) {
                 const f32x4 q = acts4[k];
-                av[4 * k] = q.x;
-                av[4 * k + 1] = q.y;
-                av[4 * k + 2] = q.z;
-                av[4 * k + 3] = q.w;
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kRows; ++k) {
-                if (r0 + k < bn) {  // rows in order, the ragged last chunk stops at A
-                    l1 += w1[k] * av[k];
-                    l2 += w2[k] * av[k];
-                }
+                if (r0 + 4 * k < bn) l1 += w1[4 * k] * q.x;  // rows in order, the ragged last chunk stops at A
+                if (r0 + 4 * k + 1 < bn) l1 += w1[4 * k + 1] * q.y;
+                if (r0 + 4 * k + 2 < bn) l1 += w1[4 * k + 2] * q.z;
+                if (r0 + 4 * k + 3 < bn) l1 += w1[4 * k + 3] * q.w;
             }
         }
-    }
-    __syncthreads();  // the latent is visible (A = 0 skips the loop's barriers)
-    // the context contribution (read from the latent in sh.aux) is computed
-    // before the neural-loss pass reuses sh.aux, and added after it
-    float c1 = 0.0f, c2 = 0.0f;
-    if (ctx_count > 0) {
-        for (uint32_t e0 = 0; e0 < E; e0 += kDims) {
-            if (e0 > 0) {
-#pragma unroll
-                for (uint32_t k = 0; k < kDims; ++k) {
-                    x1[k] = e0 + k < E ? ld(&d.p.ctx_out[o1 * E + e0 + k]) : 0.0f;
-                    x2[k] = e0 + k < E && has2 ? ld(&d.p.ctx_out[o2 * E + e0 + k]) : 0.0f;
-                }
-            }
-#pragma unroll
-            for (uint32_t k = 0; k < kDims; ++k) {
-                if (e0 + k >= E) break;
-                c1 += x1[k] * lat[e0 + k];
-                c2 += x2[k] * lat[e0 + k];
-            }
-        }
-    }
-    if (sp.flags & kStepNeuralLoss) {
-        // loss_from_logits on the neural logits, before the context is added
-        // (runtime.rs:1119, 1151-1167): f32::max fold, exp, serial sum
-        float nm = has2 ? maxnum(l1, l2) : l1;
-        for (int off = 32; off > 0; off >>= 1) nm = maxnum(nm, __shfl_xor(nm, off));
-        if (lane == 0) sh.redf[wave] = nm;
         __syncthreads();
-        nm = sh.redf[0];
-        for (uint32_t w = 1; w < kWavesPerGroup; ++w) nm = maxnum(nm, sh.redf[w]);
-        sh.aux[o1] = glibc_expf_nonpositive(l1 - nm);
-        if (has2) sh.aux[o2] = glibc_expf_nonpositive(l2 - nm);
-        __syncthreads();
-        StepRecord LEO_GLOBAL& rec = d.records[step_index];
-        if (threadIdx.x == 0) {
-            const float sum = serial_sum_outputs(sh.aux);
-            rec.neural_max = nm;
-            rec.neural_sum = sum;
-        }
-        if (sp.target_index >= 0 && static_cast<uint32_t>(sp.target_index) == o1) rec.neural_target = l1;
-        if (sp.target_index >= 0 && has2 && static_cast<uint32_t>(sp.target_index) == o2) rec.neural_target = l2;
-        __syncthreads();
+        if (end_thread)
+            for (uint32_t r = 0; r < bn; ++r) l2 += ends[r];
+        if (A > kThreads) __syncthreads();  // this block's ids and products are consumed
     }
-    if (ctx_count > 0) {
-        l1 += c1;
-        l2 += c2;
+    const bool neural = (sp.flags & kStepNeuralLoss) != 0;
+    // the neural logits' loss is taken before the context is added
+    // (runtime.rs:1119, 1151-1167)
+    const float n1 = l1, n2 = l2;
+    if (sh.ctx_cells > 0) {
+        l1 += sh.ctx_logit[o1];
+        if (end_thread) l2 += sh.ctx_logit[kEndIndex];
     }
-    sh.err[o1] = l1;
     d.logits[o1] = l1;
-    if (has2) {
-        sh.err[o2] = l2;
-        d.logits[o2] = l2;
+    if (end_thread) d.logits[kEndIndex] = l2;
+    // maxima: order-independent, reduced across the workgroup
+    const float mw = wave_max_f32(end_thread ? maxnum(l1, l2) : l1);
+    if (lane == 0) sh.redf[0][wave] = mw;
+    if (neural) {
+        const float nw = wave_max_f32(end_thread ? maxnum(n1, n2) : n1);
+        if (lane == 0) sh.redf[1][wave] = nw;
     }
-    // maximum: order-independent, reduced across the workgroup
-    float mx = has2 ? maxnum(l1, l2) : l1;
-    for (int off = 32; off > 0; off >>= 1) mx = maxnum(mx, __shfl_xor(mx, off));
-    if (lane == 0) sh.redf[wave] = mx;
     __syncthreads();
-    mx = sh.redf[0];
-    for (uint32_t w = 1; w < kWavesPerGroup; ++w) mx = maxnum(mx, sh.redf[w]);
+    float mx = sh.redf[0][0], nm = sh.redf[1][0];
+    for (uint32_t w = 1; w < kWavesPerGroup; ++w) {
+        mx = maxnum(mx, sh.redf[0][w]);
+        nm = maxnum(nm, sh.redf[1][w]);
+    }
     // exp in parallel (glibc expf), then the serial sum of runtime.rs:1175-1180
-    sh.aux[o1] = glibc_expf_nonpositive(l1 - mx);
-    if (has2) sh.aux[o2] = glibc_expf_nonpositive(l2 - mx);
+    const float x1 = glibc_expf_nonpositive(l1 - mx);
+    float x2 = 0.0f;
+    sh.aux[o1] = x1;
+    if (end_thread) sh.aux[kEndIndex] = x2 = glibc_expf_nonpositive(l2 - mx);
+    if (neural) {
+        sh.err[o1] = glibc_expf_nonpositive(n1 - nm);
+        if (end_thread) sh.err[kEndIndex] = glibc_expf_nonpositive(n2 - nm);
+    }
     __syncthreads();
-    if (threadIdx.x == 0) sh.redf[0] = serial_sum_outputs(sh.aux);
-    __syncthreads();
-    const float sum = sh.redf[0];
+    const float sum = serial_sum_outputs(sh.aux);
+    if (neural) {
+        if (wave == kWavesPerGroup - 1) {
+            const float nsum = serial_sum_outputs(sh.err);
+            if (lane == 0) {
+                rec.neural_max = nm;
+                rec.neural_sum = nsum;
+            }
+        }
+        if (static_cast<int32_t>(o1) == sp.target_index) rec.neural_target = n1;
+        if (end_thread && sp.target_index == static_cast<int32_t>(kEndIndex)) rec.neural_target = n2;
+    }
     const bool uniform = !finitef(sum) || sum <= 0.0f;
-    const float p1 = uniform ? 1.0f / static_cast<float>(kOutputs) : sh.aux[o1] / sum;
-    const float p2 = has2 ? (uniform ? 1.0f / static_cast<float>(kOutputs) : sh.aux[o2] / sum) : 0.0f;
+    const float p1 = uniform ? 1.0f / static_cast<float>(kOutputs) : x1 / sum;
+    const float p2 = uniform ? 1.0f / static_cast<float>(kOutputs) : x2 / sum;  // the end thread's
+    const float e1 = static_cast<int32_t>(o1) == sp.target_index ? p1 - 1.0f : p1;
+    const float e2 = sp.target_index == static_cast<int32_t>(kEndIndex) ? p2 - 1.0f : p2;
     d.probs[o1] = p1;
-    d.errors[o1] = static_cast<int32_t>(o1) == sp.target_index ? p1 - 1.0f : p1;
-    if (has2) {
-        d.probs[o2] = p2;
-        d.errors[o2] = static_cast<int32_t>(o2) == sp.target_index ? p2 - 1.0f : p2;
+    d.errors[o1] = e1;
+    if (static_cast<int32_t>(o1) == sp.target_index) rec.p_target = p1;
+    if (end_thread) {
+        d.probs[kEndIndex] = p2;
+        d.errors[kEndIndex] = e2;
+        if (sp.target_index == static_cast<int32_t>(kEndIndex)) rec.p_target = p2;
     }
     // argmax: largest probability, first index among equals (runtime.rs:1190-1197);
     // probabilities are non-negative, so their bit patterns order them
-    unsigned long long best = (static_cast<unsigned long long>(__float_as_uint(p1)) << 32) | (0xffffffffu - o1);
-    if (has2) {
-        const unsigned long long k2 = (static_cast<unsigned long long>(__float_as_uint(p2)) << 32) | (0xffffffffu - o2);
-        best = k2 > best ? k2 : best;
+    const uint32_t top = wave_max_u32(__float_as_uint(p1));
+    const uint64_t at_top = __ballot(__float_as_uint(p1) == top);
+    // The learning phase's bias update (runtime.rs:1290-1298), checked
+    // ahead: the reference adds the outputs' deltas in order and stops at
+    // the first bias that becomes non-finite (after writing it), before
+    // the context, synapse and homeostasis updates. The learning phase
+    // reads the first such output from the control word.
+    const bool learn = (sp.flags & kStepLearn) != 0;
+    const float olr = cfg.output_learning_rate, ss = sp.supervised_strength, mu = cfg.max_update;
+    const uint64_t bad = __ballot(learn && !finitef(bias1 + bounded(-olr * ss * e1, mu)));
+    if (lane == 0) {
+        const uint32_t first = wave * kWaveSize;
+        sh.red[0][wave] = top;
+        sh.red[1][wave] = first + static_cast<uint32_t>(__ffsll(static_cast<long long>(at_top)) - 1);
+        sh.red[2][wave] = bad ? first + static_cast<uint32_t>(__ffsll(static_cast<long long>(bad)) - 1) : kNoFail;
     }
-    best = wave_max_u64(best);
     __syncthreads();
-    if (lane == 0) sh.red[wave] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t w = 1; w < kWavesPerGroup; ++w) best = sh.red[w] > best ? sh.red[w] : best;
-        best = sh.red[0] > best ? sh.red[0] : best;
-        StepRecord& rec = d.records[step_index];
-        rec.predicted = 0xffffffffu - static_cast<uint32_t>(best);
-    }
-    if (sp.target_index >= 0 && (threadIdx.x == static_cast<uint32_t>(sp.target_index) ||
-                                 (has2 && o2 == static_cast<uint32_t>(sp.target_index))))
-        d.records[step_index].p_target = threadIdx.x == static_cast<uint32_t>(sp.target_index) ? p1 : p2;
-    __syncthreads();  // thread 0 has read the argmax partials in sh.red
-    if (sp.flags & kStepLearn) {
-        // The learning phase's bias update (runtime.rs:1290-1298), checked
-        // ahead: the reference adds the outputs' deltas in order and stops at
-        // the first bias that becomes non-finite (after writing it), before
-        // the context, synapse and homeostasis updates. The learning phase
-        // reads the first such output from the control word.
-        const float olr = cfg.output_learning_rate, ss = sp.supervised_strength, mu = cfg.max_update;
-        const float e1 = static_cast<int32_t>(o1) == sp.target_index ? p1 - 1.0f : p1;
-        const float e2 = static_cast<int32_t>(o2) == sp.target_index ? p2 - 1.0f : p2;
-        uint32_t fail = kNoFail;
-        if (!finitef(bias1 + bounded(-olr * ss * e1, mu))) fail = o1;
-        else if (has2 && !finitef(bias2 + bounded(-olr * ss * e2, mu))) fail = o2;
-        for (int off = 32; off > 0; off >>= 1) fail = min(fail, static_cast<uint32_t>(__shfl_xor(static_cast<int>(fail), off)));
-        if (lane == 0) sh.red[wave] = fail;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (uint32_t w = 1; w < kWavesPerGroup; ++w) fail = min(fail, static_cast<uint32_t>(sh.red[w]));
+    if (end_thread) {
+        uint32_t best = sh.red[0][0], where = sh.red[1][0], fail = sh.red[2][0];
+        for (uint32_t w = 1; w < kWavesPerGroup; ++w) {
+            if (sh.red[0][w] > best) {
+                best = sh.red[0][w];
+                where = sh.red[1][w];
+            }
+            fail = min(fail, sh.red[2][w]);
+        }
+        rec.predicted = __float_as_uint(p2) > best ? kEndIndex : where;
+        if (learn) {
+            if (fail == kNoFail && !finitef(bias2 + bounded(-olr * ss * e2, mu))) fail = kEndIndex;
             ctl->bias_fail = fail;
         }
     }
@@ -3050,8 +3114,7 @@ constexpr uint32_t kSignalLines = kEndIndex / 32;  // 128-byte lines before the 
 struct SignalRows {
     f32x4 line[kSignalLines];
     float tail;        // the end-class weight of the row this lane ends with
-    uint32_t dst_end;  // and that row's destination
-    bool live_end;
+    uint32_t dst_end;  // and that row's destination, ~0 past the batch's end
 };
 __device__ __forceinline__ uint32_t swap_halves(uint32_t v) {  // lanes 0-7 and 8-15 of each sixteen exchanged
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xf, 0xf, false));
@@ -3063,8 +3126,7 @@ __device__ __forceinline__ void load_signal_rows(SignalRows& r, __amdgpu_buffer_
 #pragma unroll
     for (uint32_t l = 0; l < kSignalLines; ++l) r.line[l] = ld16_record(rows, (l & 1) ? other : dst, l * 128 + seg * 16);
     r.tail = ld4_record(rows, other, 4 * kEndIndex);
-    r.dst_end = other;
-    r.live_end = swap_halves(live ? 1u : 0u) != 0;
+    r.dst_end = swap_halves(live ? dst : ~0u);
 }
 // The serial sums; lanes 7 and 15 of each sixteen return those of their dst_end.
 __device__ __forceinline__ float sum_signal_rows(const SignalRows& r, const f32x4 (&err)[kSignalLines], float err_end) {
@@ -3112,20 +3174,22 @@ __device__ __forceinline__ void phase_signals(const StepCtx& c, StepShared& sh) 
     const float err_end = sh.err[kEndIndex];
     // rows addressed by index (N records of kOutStride floats)
     const __amdgpu_buffer_rsrc_t rows = record_rsrc(d.p.out_w, kOutStride * 4, N);
-    SignalRows cur;
-    load_signal_rows(cur, rows, at < count ? dst : 0u, at < count);
-    while (true) {
+    // two sets of rows in turn (a copy from one to the other would wait for
+    // the loads); true when a batch is left
+    SignalRows r0, r1;
+    load_signal_rows(r0, rows, at < count ? dst : 0u, at < count);
+    auto batch = [&](const SignalRows& cur, SignalRows& ahead) {
         at += stride;
         const bool more = at - sub < count;  // wave-uniform
-        SignalRows ahead = cur;
         if (more) {
             load_signal_rows(ahead, rows, at < count ? next : 0u, at < count);
             next = at + stride < N ? ld(&d.dest_list[at + stride]) : 0u;
         }
         const float sig = sum_signal_rows(cur, err, err_end);
-        if ((lane & 7u) == 7u && cur.live_end) d.learning_signal[cur.dst_end] = sig;
-        if (!more) break;
-        cur = ahead;
+        if ((lane & 7u) == 7u && cur.dst_end != ~0u) d.learning_signal[cur.dst_end] = sig;
+        return more;
+    };
+    while (batch(r0, r1) && batch(r1, r0)) {
     }
 }
 
@@ -3568,6 +3632,10 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
         // the context of a step delivered ahead: on the workgroup that owns no
         // selection blocks, beside the fold (first read by the readout)
         if (delivered_ahead && c.P > 1 && c.part == c.P - 1) context_resolve(c, sp, sh);
+        if (__builtin_expect((sp.flags & kStepOutput) && c.part == c.P - 1, 0)) {
+            __syncthreads();  // the resolved cells are in LDS
+            context_logits(c, sh);
+        }
         const unsigned long long t_context = timer ? wall_clock64() : 0;
         phase_fold_select(c, sh, trace, pi, after_one_barrier);
         const unsigned long long t_fold = timer ? wall_clock64() : 0;
