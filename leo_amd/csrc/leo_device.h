@@ -477,6 +477,7 @@ struct KernelArgs {
     uint32_t profile_part;           // workgroup whose phases the profiling build times (of each lane)
     DeepSortPlan deep;
     FastDiv div_synapses;            // synapses_per_neuron
+    FastDiv div_fanout;              // input_fanout
     FastDiv div_block;               // neurons_per_block
     FastDiv div_block_words;         // block_words(neurons_per_block)
     // A tally launch (the frozen-only build, one lane, host discards the

@@ -454,6 +454,11 @@ __device__ __forceinline__ float key_activation(uint64_t key) { return __uint_as
 
 // Steps whose parameters one load round brings into LDS.
 constexpr uint32_t kStepChunk = 64;
+constexpr uint32_t kStepWords = sizeof(StepParams) / 4;
+static_assert(sizeof(StepParams) % 4 == 0 && offsetof(StepParams, symbol) == 0, "32-bit words, the symbol first");
+// Ticks whose injections a one-barrier step of a frozen-only launch may take
+// at once: one for each bucket set but the one being folded.
+constexpr uint32_t kInjectAhead = kBucketSets - 1;
 
 // Shared memory of the step kernel, reused phase by phase.
 struct alignas(16) StepShared {
@@ -511,6 +516,9 @@ struct StepCtx {
     bool local;        // workgroups of the lane share one L2 (see lane_barrier)
     bool carried;      // a one-barrier step's barrier carries the waves' winner totals
     uint32_t* tally;   // a tally launch: this wave's totals in LDS (kTally* words); else null
+    // a tally launch's per-lane counts, added to the wave's totals at its end
+    mutable uint32_t folded, inhibitory;
+    mutable uint32_t touched;  // (the wave's)
 };
 
 // This thread's item index when a phase's items are dealt 64 at a time to the
@@ -571,14 +579,12 @@ __device__ __forceinline__ uint32_t LEO_GLOBAL* counter_word(const StepCtx& c, u
 
 // Adds a wave's count to its workgroup's counter (every lane of the wave calls).
 __device__ __forceinline__ void count_wave(const StepCtx& c, uint32_t kind, uint32_t tick, uint32_t local) {
-    const uint32_t total = wave_sum_u32(local);
-    if (__lane_id() == 0 && total) {
-        if (c.tally) {
-            if (kind == kCInhibitory) c.tally[kTInhibitory] += total;
-        } else {
-            atomicAdd(counter_word(c, c.part, kind, tick), total);
-        }
+    if (c.tally) {
+        if (kind == kCInhibitory) c.inhibitory += local;
+        return;
     }
+    const uint32_t total = wave_sum_u32(local);
+    if (__lane_id() == 0 && total) atomicAdd(counter_word(c, c.part, kind, tick), total);
 }
 
 // One counter of `tick` summed over the lane's workgroups by a whole wave, uniform.
@@ -1819,14 +1825,16 @@ __device__ __forceinline__ void phase_fold_select(const StepCtx& c, StepShared& 
         }
     }
     const uint32_t listed_before = listed - b0 * nb;
-    entries = wave_sum_u32(entries);
+    if (c.tally) {
+        // no counter atomics mid-step: each would hold up the wave's later
+        // load waits (memory operations retire in order)
+        c.folded += entries;
+        c.touched += listed_before;
+    } else {
+        entries = wave_sum_u32(entries);
+    }
     if (lane == 0) {
-        if (c.tally) {
-            // no counter atomics mid-step: each would hold up the wave's later
-            // load waits (memory operations retire in order)
-            c.tally[kTEvents] += entries;
-            c.tally[kTTouched] += listed_before;
-        } else {
+        if (!c.tally) {
             if (supra) atomicAdd(counter_word(c, c.part, kCSupra, tick), supra);
             if (entries) atomicAdd(counter_word(c, c.part, kCEvents, tick), entries);
             if (listed_before) atomicAdd(counter_word(c, c.part, kCTouched, tick), listed_before);
@@ -2065,7 +2073,45 @@ __device__ __forceinline__ void write_active(const StepCtx& c, const StepParams&
 // stale tick there and deliver nothing from it: every event of t is
 // already in its bucket).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, uint32_t early, const StepParams& next) {
+//
+// The injections of the next `inject` ticks (frozen steps of this launch, all
+// one-barrier: their sets are free) go out together, every kInjectAhead steps
+// in a frozen-only launch: 64 items a wave on every workgroup once, where a
+// tick's own F items kept the first waves of a few workgroups, which then
+// ended the phase, busy in every step (claims and stores of ~1.2 us at 512
+// items). Step-kernel time at a million units, 470 frozen and 32 learning
+// steps: 7.07 -> 6.75 ms; a batch at 16,384 units 362 -> 345 ms. A lane reads
+// the ring's bookkeeping only while a two-phase tick can still have left
+// events there. `symbols`: the LDS step parameters from the next step on. `ring`: earlier two-phase ticks may have left events of
+// the next tick in the ring.
+struct Injection {
+    bool live;
+    uint32_t target, tick;
+    uint64_t key;
+    float value;
+};
+__device__ __forceinline__ Injection fetch_injection(const StepCtx& c, const uint32_t* symbols, uint32_t item,
+                                                     uint32_t items) {
+    Injection in{};
+    in.live = item < items;
+    if (in.live) {
+        const uint32_t F = c.a->cfg.input_fanout;
+        const uint32_t ahead = fast_div(item, c.a->div_fanout), i = item - ahead * F;
+        const uint64_t slot = static_cast<uint64_t>(symbols[ahead * kStepWords]) * F + i;
+        const uint32_t edge = c.a->m.in_edge[slot];  // target and branch in one load
+        in.value = ld(&c.d.p.in_weight[slot]);
+        in.target = edge_target(edge);
+        in.key = (4ULL << 61) | (static_cast<uint64_t>(i) << 2) | edge_branch(edge);
+        in.tick = c.tick + 1 + ahead;
+    }
+    return in;
+}
+__device__ __forceinline__ void write_injection(const StepCtx& c, const Injection& in, const EntryClaim& k) {
+    if (write_entry(c, set_of(c.d, in.tick), in.target, k, in.key, in.value)) touch_neuron(c, in.target, in.tick);
+}
+
+__device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, uint32_t early, const StepParams& next,
+                                            const uint32_t* symbols, uint32_t inject, bool ring) {
     const LeoConfig& cfg = c.a->cfg;
     const LaneDesc& d = c.d;
     const uint32_t wave = wave_index(), lane = __lane_id();
@@ -2075,12 +2121,11 @@ __device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, ui
     const uint32_t b0 = min(cfg.block_count, wv * range);
     const uint64_t row0 = static_cast<uint64_t>(b0) * cfg.max_active_per_block;
     const uint32_t S = cfg.synapses_per_neuron;
-    // tick t+1's other deliveries, dealt over every workgroup: this thread's
-    // first item's loads go out before the winners' work
-    const DeliverPlan np = deliver_plan(c, sh, true);
-    const uint32_t dealt = dealt_index(c, c.P);
-    DeliverItem item0 = deliver_fetch(c, next, np, np.delivers ? dealt : np.total);
-    reset_next_lists(c);
+    // dealt over every workgroup: this thread's first injection's loads go out
+    // before the winners' work
+    const uint32_t dealt = dealt_index(c, c.P), injections = inject * cfg.input_fanout;
+    Injection in0{};
+    if (inject) in0 = fetch_injection(c, symbols, dealt, injections);
     const uint32_t mine = sh.win_count[wave];
     // staged winners past the wave's LDS copy are read back from memory the
     // wave has just written
@@ -2110,14 +2155,10 @@ __device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, ui
     // phase's prologue fills. A lane takes up to kEmitBatch events per round
     // of memory operations (their synapse loads, then their bucket claims,
     // then their entry writes), and the first round also claims the bucket
-    // entry of its next-tick injection, whose loads went out above.
+    // entry of its first injection, whose loads went out above.
     constexpr uint32_t kEmitBatch = 4;
     const uint32_t items = early ? mine * S : 0u;
-    const bool inj0 = np.delivers && item0.inj;
-    const uint32_t inj_set = set_of(d, c.tick + 1);
-    const uint32_t rounds = items > 0 ? (items + kEmitBatch * kWaveSize - 1) / (kEmitBatch * kWaveSize) : 1u;
-    for (uint32_t round = 0; round < rounds; ++round) {
-        const uint32_t base = round * kEmitBatch * kWaveSize;
+    for (uint32_t base = 0; base < items || (base == 0 && inject); base += kEmitBatch * kWaveSize) {
         uint32_t edge[kEmitBatch], rj[kEmitBatch];
         float value[kEmitBatch];
         bool live[kEmitBatch];
@@ -2149,8 +2190,8 @@ __device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, ui
             if (live[k]) claim[k] = claim_entry(c, set[k], edge_target(edge[k]));
         }
         EntryClaim inj{};
-        const bool inj_here = round == 0 && inj0;
-        if (inj_here) inj = claim_entry(c, inj_set, item0.target);
+        const bool inj_here = base == 0 && in0.live;
+        if (inj_here) inj = claim_entry(c, set_of(d, in0.tick), in0.target);
 #pragma unroll
         for (uint32_t k = 0; k < kEmitBatch; ++k) {
             if (!live[k]) continue;
@@ -2161,13 +2202,18 @@ __device__ __forceinline__ void frozen_emit(const StepCtx& c, StepShared& sh, ui
             if (write_entry(c, set[k], edge_target(edge[k]), claim[k], key, value[k]))
                 touch_neuron(c, edge_target(edge[k]), c.tick + (1u << dl));
         }
-        if (inj_here && write_entry(c, inj_set, item0.target, inj, item0.key, item0.value))
-            touch_neuron(c, item0.target, c.tick + 1);
+        if (inj_here) write_injection(c, in0, inj);
     }
-    uint32_t delivered = 0;  // counted by the fold
-    item0.inj = item0.inj && !inj0;  // an injection claimed above is done
-    if (np.delivers) deliver_commit(c, next, np, item0, delivered);
-    deliver_items(c, next, np, dealt + np.stride, delivered);
+    for (uint32_t item = dealt + c.gstride; item - lane < injections; item += c.gstride) {
+        const Injection in = fetch_injection(c, symbols, item, injections);
+        if (in.live) write_injection(c, in, claim_entry(c, set_of(d, in.tick), in.target));
+    }
+    if (ring) {
+        DeliverPlan np = deliver_plan(c, sh, true);
+        np.total = np.off_in;  // the ring's items without the injection
+        uint32_t delivered = 0;  // counted by the fold
+        deliver_items(c, next, np, dealt, delivered);
+    }
     count_wave(c, kCInhibitory, c.tick, inhibitory);
 }
 
@@ -3514,6 +3560,7 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
     // per-step counter words, which the launch leaves untouched, for the
     // lane's next launch.
     c.tally = nullptr;
+    c.folded = c.inhibitory = c.touched = 0;
     if (kFrozenOnly && args.tally) {
         c.tally = &sh.tally[wave_index()][0];
         if (threadIdx.x < kWavesPerGroup * kTWaveWords) (&sh.tally[0][0])[threadIdx.x] = 0u;
@@ -3562,8 +3609,6 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
     // of coalesced loads into LDS: a load per step, even issued a step
     // ahead, would be waited for by the step's first wait on its own loads
     // (the vector memory counter drains in order)
-    constexpr uint32_t kStepWords = sizeof(StepParams) / 4;
-    static_assert(sizeof(StepParams) % 4 == 0, "step parameters are 32-bit words");
     uint32_t chunk_base = 0;
     auto load_chunk = [&](uint32_t first) {
         chunk_base = first;
@@ -3592,6 +3637,8 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
     bool delivered_ahead = false, stopped = false, after_one_barrier = false;
     float pi_read = 0.0f;
     uint32_t early_prev = 0;  // kStepEarly delays of the one-barrier step before
+    uint32_t injected = 0;    // coming ticks whose injections have gone out
+    uint32_t quiet = 0;       // one-barrier steps in a row that left the ring nothing
     const bool one_barrier_lane = c.d.bucket_sets != 1 && c.P > 1 && redundant;
     for (uint32_t s = 0; s < steps && ok; ++s) {
         if (s % kStepChunk == 0) load_chunk(s);
@@ -3658,7 +3705,19 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
                 clock.section(4, t_prologue, t_context);
                 clock.section(5, t_context, t_fold);
             }
-            frozen_emit(c, sh, early_prev, next);
+            // the injections of the coming ticks in one go: a frozen-only
+            // launch's steps but the last are all one-barrier, and the step
+            // parameters at hand give their symbols
+            uint32_t inject = 0;
+            if (injected == 0) {
+                inject = kFrozenOnly ? min(kInjectAhead, min(steps - 1 - s, chunk_base + kStepChunk - s)) : 1u;
+                injected = inject;
+            }
+            injected -= 1;
+            // ring events of tick+1 come from ticks up to seven before this one
+            frozen_emit(c, sh, early_prev, next, &sh.step_chunk[(s + 1 - chunk_base) * kStepWords], inject, quiet < 7);
+            if (!kFrozenOnly) reset_next_lists(c);
+            quiet = early_prev == (kStepEarlyMask >> kStepEarlyShift) ? quiet + 1 : 0;
             // after a two-phase step, the roll its successor's active-list
             // phase would make: that step's record is finished and the
             // counters tick+1 reuses are cleared (a one-barrier step's
@@ -3672,6 +3731,7 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
             c.tick += 1;
             continue;
         }
+        quiet = 0;
         if (!(ok = phase_barrier<kProfile>(c, target, spin, clock, 1))) break;
         // An output step's readout runs on the last workgroup beside the
         // eligibility update, which the other workgroups share (a lane of one
@@ -3721,10 +3781,15 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
     }
     if (ok && !stopped && !c.tally && c.part == 0 && threadIdx.x < kWaveSize && steps > 0)
         finalize_record(c, steps - 1, c.tick - 1);
+    const uint32_t folded = c.tally ? wave_sum_u32(c.folded) : 0u;
+    const uint32_t inhibitory = c.tally ? wave_sum_u32(c.inhibitory) : 0u;
     if (ok && c.tally && __lane_id() == 0) {
         // each wave's totals; the recording wave's 64-bit sums (it is the
         // only writer of those words after the launch's first barrier)
         const uint32_t wave = wave_index();
+        sh.tally[wave][kTEvents] += folded;
+        sh.tally[wave][kTTouched] += c.touched;
+        sh.tally[wave][kTInhibitory] += inhibitory;
 #pragma unroll
         for (uint32_t k = 0; k < kTWaveWords; ++k)
             if (sh.tally[wave][k]) atomicAdd(&args.tally[k], sh.tally[wave][k]);

@@ -704,6 +704,7 @@ KernelArgs kernel_args(LeoHipRuntime* h, LaneDesc* lanes, uint32_t count, uint32
     a.lane_stride = count;
     a.local_sync = h->local_sync ? 1 : 0;
     a.div_synapses = make_fast_div(h->cfg.device.synapses_per_neuron);
+    a.div_fanout = make_fast_div(h->cfg.device.input_fanout);
     a.div_block = make_fast_div(h->cfg.device.neurons_per_block);
     a.div_block_words = make_fast_div(block_words(h->cfg.device.neurons_per_block));
     a.skip_zero_eligibility = h->negative_zero_weights ? 0u : 1u;
