@@ -164,17 +164,21 @@ enum : uint32_t {
 };
 constexpr uint32_t kNoFail = 0xffffffffu;
 
+struct alignas(8) ListCounts {
+    uint32_t kept;   // entries of the eligible list
+    uint32_t learn;  // entries of the step's learning-slot list
+};
+
 // Device-resident scalars of a lane that persist across launches.
 struct LaneControl {
     uint32_t tick;                   // current_tick
     float population_inhibition;
     uint32_t parity;                 // which eligible list is current
-    uint32_t rec_count[2];
-    uint32_t in_count[2];
+    // by parity: the lengths of an eligible list and of the learning-slot list
+    // written with it, one 64-bit word, so that one atomic reserves both
+    ListCounts rec_list[2], in_list[2];
     uint32_t dest_epoch;             // learning-destination epoch
     uint32_t dest_count;             // entries of this step's destination list
-    uint32_t rec_learn_count;        // entries of this step's recurrent learning-slot list
-    uint32_t in_learn_count;         // entries of this step's input learning-slot list
     uint32_t history_len;
     uint32_t history[kMaxOrder];
     uint32_t ctx_count;
@@ -305,8 +309,8 @@ struct LaneDesc {
     uint32_t LEO_GLOBAL* dest_list;     // N: this step's claimed learning destinations (LaneControl dest_count)
     // this step's learning slots: kept eligible slots whose weight update can
     // change the weight (nonzero eligibility), listed by the eligibility phase
-    uint32_t LEO_GLOBAL* rec_learn;     // NS (LaneControl rec_learn_count)
-    uint32_t LEO_GLOBAL* in_learn;      // NI (LaneControl in_learn_count)
+    uint32_t LEO_GLOBAL* rec_learn;     // NS (LaneControl rec_list.learn)
+    uint32_t LEO_GLOBAL* in_learn;      // NI (LaneControl in_list.learn)
     // Delivery buckets in bucket_sets sets (1, or kBucketSets on a lane that
     // takes frozen runs with one barrier per step): the deliveries of tick t
     // go to set t % bucket_sets, so events emitted up to 8 ticks ahead wait

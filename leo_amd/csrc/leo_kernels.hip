@@ -907,9 +907,9 @@ __device__ __forceinline__ void deliver_commit(const StepCtx& c, const StepParam
     uint8_t LEO_GLOBAL* mark = it.ring ? d.rec_mark + rslot : d.in_mark + it.slot;
     if (fresh) *mark = kMarkListed;
     const bool new_rec = fresh && it.ring, new_in = fresh && !it.ring;
-    uint32_t pos = wave_append(&ctl->rec_count[c.parity], new_rec);
+    uint32_t pos = wave_append(&ctl->rec_list[c.parity].kept, new_rec);
     if (new_rec) d.rec_list[static_cast<uint64_t>(c.parity) * NS + pos] = eslot;
-    pos = wave_append(&ctl->in_count[c.parity], new_in);
+    pos = wave_append(&ctl->in_list[c.parity].kept, new_in);
     if (new_in) d.in_list[static_cast<uint64_t>(c.parity) * NI + pos] = eslot;
 }
 
@@ -926,8 +926,8 @@ __device__ __forceinline__ void deliver_items(const StepCtx& c, const StepParams
 // Reset of this step's next eligible lists (trace steps append to them).
 __device__ __forceinline__ void reset_next_lists(const StepCtx& c) {
     if (c.part == 0 && threadIdx.x == 0) {
-        c.ctl->rec_count[c.parity ^ 1] = 0;
-        c.ctl->in_count[c.parity ^ 1] = 0;
+        c.ctl->rec_list[c.parity ^ 1] = ListCounts{0, 0};
+        c.ctl->in_list[c.parity ^ 1] = ListCounts{0, 0};
     }
 }
 
@@ -1890,8 +1890,8 @@ __device__ __forceinline__ void write_active(const StepCtx& c, const StepParams&
     if (recorder) {
         pi_old = ld(&c.ctl->population_inhibition);
         if (fuse_post) {
-            rec_n = ld(&c.ctl->rec_count[c.parity]);
-            in_n = ld(&c.ctl->in_count[c.parity]);
+            rec_n = ld(&c.ctl->rec_list[c.parity].kept);
+            in_n = ld(&c.ctl->in_list[c.parity].kept);
             // the context of this step is resolved (phase 1 or 2); the next
             // step's resolution runs after these loads (phase 2 of the next
             // step, or below on the same workgroup)
@@ -2293,7 +2293,7 @@ __device__ __forceinline__ float frozen_prologue(const StepCtx& c, StepShared& s
         }
         if (lane == 0) {
             LaneControl LEO_GLOBAL* ctl = c.ctl;
-            const uint32_t rec_n = ld(&ctl->rec_count[c.parity]), in_n = ld(&ctl->in_count[c.parity]);
+            const uint32_t rec_n = ld(&ctl->rec_list[c.parity].kept), in_n = ld(&ctl->in_list[c.parity].kept);
             const uint32_t cells = ld(&ctl->ctx_count), probes = ld(&ctl->ctx_probes);
             const uint32_t applied = ld(&ctl->ctx_applied);
             if (c.tally) {
@@ -2590,68 +2590,57 @@ __device__ __forceinline__ bool finish_slot(const StepCtx& c, const SlotInputs& 
 // destinations (runtime.rs:1214-1243).
 struct LearnOut {
     uint32_t LEO_GLOBAL* list;   // learning slots of this list
-    uint32_t LEO_GLOBAL* count;
     bool plastic;                // the step commits recurrent/input plasticity
     uint32_t claimed;            // this thread's destinations claimed
     uint32_t listed;             // this thread's learning slots listed
 };
 
-// Wave-aggregated append of K predicates per lane (every lane active): one
-// atomic for the wave; lane order within each predicate, predicate k's
-// entries before predicate k+1's.
-template <uint32_t K>
-__device__ __forceinline__ void wave_append_k(uint32_t LEO_GLOBAL* counter, const bool (&p)[K], uint32_t (&pos)[K]) {
-    unsigned long long m[K];
-    uint32_t total = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < K; ++k) {
-        m[k] = __ballot(p[k]);
-        total += static_cast<uint32_t>(__popcll(m[k]));
-    }
-    uint32_t base = 0;
-    if (total != 0 && __lane_id() == 0) base = atomicAdd(counter, total);
-    base = __builtin_amdgcn_readfirstlane(base);
-    const unsigned long long below = (1ULL << __lane_id()) - 1ULL;
-#pragma unroll
-    for (uint32_t k = 0; k < K; ++k) {
-        pos[k] = base + static_cast<uint32_t>(__popcll(m[k] & below));
-        base += static_cast<uint32_t>(__popcll(m[k]));
-    }
-}
-
-// Eligible slots of one list, K per lane per iteration (their loads in
-// flight together: 2 when the list gives each thread a few slots, more when
-// it gives each many, as on story lanes with few workgroups); kept slots are
-// compacted into the next list. On a
-// plasticity step the kept slots whose update can change their weight
-// (nonzero eligibility; every kept slot when skip_zero_eligibility is off) are
-// listed as learning slots, and their destinations are claimed once each
-// with an epoch exchange: the learning signal is computed for exactly those.
-// The reference also computes signals for the other destinations (the
-// targets of zero-eligibility slots and the active neurons); no update reads
-// them.
+// Eligible slots of one list, K per lane per iteration (their loads in flight
+// together); kept slots are compacted into the next list. On a plasticity step
+// the kept slots whose update can change their weight (nonzero eligibility;
+// every kept slot when skip_zero_eligibility is off) are listed as learning
+// slots, and their destinations are claimed once each with an epoch exchange:
+// the learning signal is computed for exactly those. The reference also
+// computes signals for the other destinations (the targets of zero-eligibility
+// slots and the active neurons); no update reads them.
 // Each slot's packed synapse (`edges`) gives its destination and branch in
-// one load.
+// one load. An iteration is a chain of memory rounds: slots (loaded an
+// iteration ahead), records and synapses, touched words, touched
+// destinations; then one atomic reserves the places in both lists (`counts`)
+// together with the destination claims, and one the claimed destinations'
+// places. Three reservations one after the other with the claims between them
+// were four rounds: a million units' 8-lane story pass 12.9 ms then, 12.3 now
+// (with the wider iterations of eligibility_width); 16,384 and 131,072 units
+// within noise. Pairs of lanes reading and writing whole 32-byte records took
+// 11% off this phase with 32 lanes but 4% more of a single lane's step, and
+// are not used.
 template <uint32_t K>
 __device__ __forceinline__ void eligibility_list(const StepCtx& c, float LEO_GLOBAL* trace, uint64_t slots,
                                                  uint8_t LEO_GLOBAL* marks,
                                                  const uint32_t LEO_GLOBAL* cur, uint32_t cur_n,
-                                                 uint32_t LEO_GLOBAL* next, uint32_t LEO_GLOBAL* next_count,
+                                                 uint32_t LEO_GLOBAL* next, ListCounts LEO_GLOBAL* counts,
                                                  const uint32_t* edges, float pop_cutoff, LearnOut& learn,
                                                  uint32_t gstride) {
     const bool skip_zero = c.a->skip_zero_eligibility != 0;
     const uint32_t lane = __lane_id();
     const __amdgpu_buffer_rsrc_t rsrc = trace_rsrc(trace, slots);
-    for (uint32_t base = dealt_index(c, gstride / kThreads) - lane; base < cur_n; base += K * gstride) {
+    const unsigned long long below = (1ULL << lane) - 1ULL;
+    uint32_t base = dealt_index(c, gstride / kThreads) - lane;
+    uint32_t ahead[K];
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+        const uint32_t i = base + k * gstride + lane;
+        ahead[k] = i < cur_n ? ld(&cur[i]) : 0u;
+    }
+    for (; base < cur_n; base += K * gstride) {
         bool v[K];
         uint32_t sl[K], t[K];
         uint8_t r[K];
         SlotInputs in[K];
 #pragma unroll
         for (uint32_t k = 0; k < K; ++k) {
-            const uint32_t i = base + k * gstride + lane;
-            v[k] = i < cur_n;
-            sl[k] = v[k] ? ld(&cur[i]) : 0u;
+            v[k] = base + k * gstride + lane < cur_n;
+            sl[k] = ahead[k];
             t[k] = 0;
             r[k] = 0;
             in[k] = SlotInputs{};
@@ -2666,56 +2655,78 @@ __device__ __forceinline__ void eligibility_list(const StepCtx& c, float LEO_GLO
             }
         }
 #pragma unroll
+        for (uint32_t k = 0; k < K; ++k) {
+            const uint32_t i = base + (K + k) * gstride + lane;
+            ahead[k] = i < cur_n ? ld(&cur[i]) : 0u;
+        }
+#pragma unroll
         for (uint32_t k = 0; k < K; ++k)
             if (v[k]) load_touched(in[k], c, t[k]);
 #pragma unroll
         for (uint32_t k = 0; k < K; ++k)
             if (v[k] && in[k].touched_epoch == c.tick + 1) load_destination(in[k], c, t[k]);
-        float e[K];
-        bool kept[K];
+        bool kept[K], l[K];
+        unsigned long long km[K], lm[K];
+        uint32_t kept_total = 0, learn_total = 0;
 #pragma unroll
         for (uint32_t k = 0; k < K; ++k) {
-            e[k] = 0.0f;
-            kept[k] = v[k] && finish_slot(c, in[k], trace, sl[k], r[k], pop_cutoff, e[k]);
+            float e = 0.0f;
+            kept[k] = v[k] && finish_slot(c, in[k], trace, sl[k], r[k], pop_cutoff, e);
+            l[k] = learn.plastic && kept[k] && (e != 0.0f || !skip_zero);
+            km[k] = __ballot(kept[k]);
+            lm[k] = __ballot(l[k]);
+            kept_total += static_cast<uint32_t>(__popcll(km[k]));
+            learn_total += static_cast<uint32_t>(__popcll(lm[k]));
+        }
+        unsigned long long reserved = 0;
+        if (kept_total != 0 && lane == 0)
+            reserved = atomicAdd(reinterpret_cast<unsigned long long*>(counts),
+                                 (static_cast<unsigned long long>(learn_total) << 32) | kept_total);
+        uint32_t claim[K];
+#pragma unroll
+        for (uint32_t k = 0; k < K; ++k) {
+            claim[k] = c.dest_epoch;
+            if (l[k]) claim[k] = atomicExch(nu(c.d, t[k], kNDestEpoch), c.dest_epoch);
         }
 #pragma unroll
         for (uint32_t k = 0; k < K; ++k)
             if (v[k] && !kept[k]) marks[sl[k]] = kMarkDropped;
-        uint32_t pos[K];
-        wave_append_k<K>(next_count, kept, pos);
+        unsigned long long wm[K];
+        uint32_t claimed_total = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < K; ++k)
-            if (kept[k]) next[pos[k]] = sl[k];
-        if (learn.plastic) {  // wave-uniform
-            bool l[K];
+        for (uint32_t k = 0; k < K; ++k) {
+            wm[k] = __ballot(claim[k] != c.dest_epoch);
+            claimed_total += static_cast<uint32_t>(__popcll(wm[k]));
+        }
+        uint32_t dest_at = 0;
+        if (claimed_total != 0 && lane == 0) dest_at = atomicAdd(&c.ctl->dest_count, claimed_total);
+        uint32_t kept_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reserved));
+        uint32_t learn_at = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(reserved >> 32));
 #pragma unroll
-            for (uint32_t k = 0; k < K; ++k) l[k] = kept[k] && (e[k] != 0.0f || !skip_zero);
-            wave_append_k<K>(learn.count, l, pos);
+        for (uint32_t k = 0; k < K; ++k) {
+            if (kept[k]) next[kept_at + static_cast<uint32_t>(__popcll(km[k] & below))] = sl[k];
+            if (l[k]) learn.list[learn_at + static_cast<uint32_t>(__popcll(lm[k] & below))] = sl[k];
+            kept_at += static_cast<uint32_t>(__popcll(km[k]));
+            learn_at += static_cast<uint32_t>(__popcll(lm[k]));
+            learn.listed += l[k] ? 1u : 0u;
+        }
+        dest_at = __builtin_amdgcn_readfirstlane(dest_at);
 #pragma unroll
-            for (uint32_t k = 0; k < K; ++k)
-                if (l[k]) learn.list[pos[k]] = sl[k];
-            bool w[K];
-#pragma unroll
-            for (uint32_t k = 0; k < K; ++k)
-                w[k] = l[k] && atomicExch(nu(c.d, t[k], kNDestEpoch), c.dest_epoch) != c.dest_epoch;
-            wave_append_k<K>(&c.ctl->dest_count, w, pos);
-#pragma unroll
-            for (uint32_t k = 0; k < K; ++k) {
-                if (w[k]) c.d.dest_list[pos[k]] = t[k];
-                learn.listed += l[k] ? 1u : 0u;
-                learn.claimed += w[k] ? 1u : 0u;
-            }
+        for (uint32_t k = 0; k < K; ++k) {
+            const bool won = claim[k] != c.dest_epoch;
+            if (won) c.d.dest_list[dest_at + static_cast<uint32_t>(__popcll(wm[k] & below))] = t[k];
+            dest_at += static_cast<uint32_t>(__popcll(wm[k]));
+            learn.claimed += won ? 1u : 0u;
         }
     }
 }
 
 // Slots per lane and iteration for a list of n slots over gstride threads:
-// four once every thread has at least eight slots (two iterations of four
-// instead of four of two), else two (wider iterations cost a lane with only a
-// few slots more than they save: +0.5 us per supervised canonical step).
+// four when two a thread would take a second iteration, else two (a wider
+// iteration costs a lane with one or two slots more than it saves).
 template <class F>
 __device__ __forceinline__ void eligibility_width(uint32_t n, uint32_t gstride, F&& walk) {
-    if (n >= 8u * gstride) walk(std::integral_constant<uint32_t, 4>{});
+    if (n > 2u * gstride) walk(std::integral_constant<uint32_t, 4>{});
     else walk(std::integral_constant<uint32_t, 2>{});
 }
 
@@ -2728,22 +2739,22 @@ __device__ __forceinline__ void phase_eligibility(const StepCtx& c, bool plastic
     const uint64_t NS = static_cast<uint64_t>(cfg.neuron_count) * cfg.synapses_per_neuron;
     const uint64_t NI = static_cast<uint64_t>(kSymbols) * cfg.input_fanout;
     const uint32_t p = c.parity, q = c.parity ^ 1;
-    const uint32_t rec_n = ld(&c.ctl->rec_count[p]), in_n = ld(&c.ctl->in_count[p]);
+    const uint32_t rec_n = ld(&c.ctl->rec_list[p].kept), in_n = ld(&c.ctl->in_list[p].kept);
     if (c.part == 0 && threadIdx.x == 0) {
         *counter_word(c, 0, kCScanRec, c.tick) = rec_n;
         *counter_word(c, 0, kCScanIn, c.tick) = in_n;
     }
     const float pop_cutoff = a.redundant_global ? 0.0f : ld(&c.ctl->pop_cutoff);
-    LearnOut rec{d.rec_learn, &c.ctl->rec_learn_count, plastic, 0, 0};
+    LearnOut rec{d.rec_learn, plastic, 0, 0};
     eligibility_width(rec_n, gstride, [&](auto width) {
         eligibility_list<decltype(width)::value>(c, d.rec_trace, NS, d.rec_mark, d.rec_list + p * NS, rec_n,
-                                                 d.rec_list + q * NS, &c.ctl->rec_count[q], a.m.rec_edge,
+                                                 d.rec_list + q * NS, &c.ctl->rec_list[q], a.m.rec_edge,
                                                  pop_cutoff, rec, gstride);
     });
-    LearnOut in{d.in_learn, &c.ctl->in_learn_count, plastic, rec.claimed, rec.listed};
+    LearnOut in{d.in_learn, plastic, rec.claimed, rec.listed};
     eligibility_width(in_n, gstride, [&](auto width) {
         eligibility_list<decltype(width)::value>(c, d.in_trace, NI, d.in_mark, d.in_list + p * NI, in_n,
-                                                 d.in_list + q * NI, &c.ctl->in_count[q], a.m.in_edge,
+                                                 d.in_list + q * NI, &c.ctl->in_list[q], a.m.in_edge,
                                                  pop_cutoff, in, gstride);
     });
     if (plastic) {
@@ -3111,7 +3122,7 @@ __device__ __forceinline__ void phase_post(const StepCtx& c, const StepParams& s
             const uint32_t selected = ld(&ctl->block_selected);
             const uint32_t clipped = ld(&ctl->clipped), cells = ld(&ctl->ctx_count);
             const uint32_t probes = ld(&ctl->ctx_probes), applied = ld(&ctl->ctx_applied);
-            const uint32_t rec_n = ld(&ctl->rec_count[c.parity]), in_n = ld(&ctl->in_count[c.parity]);
+            const uint32_t rec_n = ld(&ctl->rec_list[c.parity].kept), in_n = ld(&ctl->in_list[c.parity].kept);
             StepRecord LEO_GLOBAL& rec = d.records[step_index];
             if (!(sp.flags & kStepOutput)) {  // an output step's readout has set them
                 rec.p_target = 0.0f;
@@ -3343,8 +3354,8 @@ __device__ __forceinline__ void phase_learn(const StepCtx& c, const StepParams& 
         // known are masked by the loops below)
         const uint32_t* rec_cur = d.rec_learn;
         const uint32_t* in_cur = d.in_learn;
-        const uint32_t rec_n = plastic ? ld(&ctl->rec_learn_count) : 0u;
-        const uint32_t in_n = plastic ? ld(&ctl->in_learn_count) : 0u;
+        const uint32_t rec_n = plastic ? ld(&ctl->rec_list[c.parity].learn) : 0u;
+        const uint32_t in_n = plastic ? ld(&ctl->in_list[c.parity].learn) : 0u;
         const uint32_t rec_first = plastic && first < NS ? ld(&rec_cur[first]) : 0u;
         const uint32_t in_first = plastic && first < NI ? ld(&in_cur[first]) : 0u;
         for (uint32_t o = threadIdx.x; o < kOutputs; o += kThreads) sh.err[o] = ld(&d.errors[o]);
@@ -3659,11 +3670,7 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
         const bool plastic = learn && sp.plasticity_scale > 0.0f;
         if (plastic) {
             c.dest_epoch += 1;
-            if (c.part == 0 && threadIdx.x == 0) {
-                c.ctl->dest_count = 0;
-                c.ctl->rec_learn_count = 0;
-                c.ctl->in_learn_count = 0;
-            }
+            if (c.part == 0 && threadIdx.x == 0) c.ctl->dest_count = 0;
         }
         // the previous tick's record and population inhibition after a
         // one-barrier frozen step (before this step's context replaces the
@@ -4003,8 +4010,8 @@ __global__ void __launch_bounds__(kThreads) leo_reset_lanes(KernelArgs args, uin
         ctl->tick = tick;
         ctl->population_inhibition = 0.0f;
         ctl->parity = 0;
-        ctl->rec_count[0] = ctl->rec_count[1] = 0;
-        ctl->in_count[0] = ctl->in_count[1] = 0;
+        ctl->rec_list[0] = ctl->rec_list[1] = ListCounts{0, 0};
+        ctl->in_list[0] = ctl->in_list[1] = ListCounts{0, 0};
         ctl->history_len = 0;
         ctl->ctx_count = 0;
         ctl->ctx_probes = 0;
@@ -4014,8 +4021,6 @@ __global__ void __launch_bounds__(kThreads) leo_reset_lanes(KernelArgs args, uin
         ctl->pop_cutoff = 0.0f;
         ctl->active_count = 0;
         ctl->dest_count = 0;
-        ctl->rec_learn_count = 0;
-        ctl->in_learn_count = 0;
         ctl->barrier = 0;
         ctl->abort = 0;
         for (uint32_t k = 0; k < kRing; ++k) {

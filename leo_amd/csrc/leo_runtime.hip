@@ -3239,13 +3239,13 @@ int32_t leo_hip_read_list(LeoHipRuntime* h, int32_t which, uint64_t* out, uint64
                 break;
             }
             case LEO_LIST_ELIGIBLE_REC: {
-                uint32_t n = ctl.rec_count[ctl.parity];
+                uint32_t n = ctl.rec_list[ctl.parity].kept;
                 v.resize(n);
                 leo::download(v.data(), d.rec_list + static_cast<uint64_t>(ctl.parity) * h->z.ns, n * 4, h->stream);
                 break;
             }
             case LEO_LIST_ELIGIBLE_IN: {
-                uint32_t n = ctl.in_count[ctl.parity];
+                uint32_t n = ctl.in_list[ctl.parity].kept;
                 v.resize(n);
                 leo::download(v.data(), d.in_list + static_cast<uint64_t>(ctl.parity) * h->z.ni, n * 4, h->stream);
                 break;
