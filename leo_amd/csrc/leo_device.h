@@ -594,6 +594,38 @@ struct FoldArgs {
 };
 enum : uint32_t { kMergeDirect = 0, kMergeAccumulate = 1, kMergeFinalize = 2 };
 
+// The host mirror's synchronisation: the elements of the five change sets
+// (threshold, recurrent, input, output rows, context slots) that are marked
+// changed or host-stale, counted and then listed (list[] null: counted only).
+constexpr uint32_t kChangeSets = 5;
+struct ChangeSets {
+    const uint32_t LEO_GLOBAL* changes[kChangeSets];
+    const uint32_t LEO_GLOBAL* stale[kChangeSets];
+    uint64_t size[kChangeSets];                          // elements
+    unsigned long long LEO_GLOBAL* count;                // per set: elements, or the list's cursor
+    uint32_t LEO_GLOBAL* list[kChangeSets];
+};
+// `count` listed output rows, transposed: out[o * count + k] is output o of
+// row list[k], so that the host writes one output's row of its output-major
+// mirror at a time.
+constexpr uint32_t kTransposeRows = 32;
+struct GatherRows {
+    const float LEO_GLOBAL* rows;
+    const uint32_t LEO_GLOBAL* list;
+    float LEO_GLOBAL* out;
+    uint64_t count;
+};
+// `count` listed context slots: keys, observations and embedding rows.
+struct GatherSlots {
+    LaneParams p;
+    const uint32_t LEO_GLOBAL* list;
+    uint64_t count;
+    uint32_t E;
+    uint64_t LEO_GLOBAL* keys;
+    uint32_t LEO_GLOBAL* obs;
+    float LEO_GLOBAL* emb;
+};
+
 }  // namespace leo
 
 #endif

@@ -4227,4 +4227,67 @@ __global__ void __launch_bounds__(kThreads) leo_fold_changes(FoldArgs f) {
     }
 }
 
+// Counts or lists the marked elements of every change set (one set per
+// blockIdx.y, one bitmap word per thread, one atomic per wave). The lists'
+// order is that of the waves' atomics; every element is moved on its own.
+__global__ void __launch_bounds__(kThreads) leo_list_changes(ChangeSets s) {
+    const uint32_t set = blockIdx.y, lane = __lane_id();
+    const uint64_t words = (s.size[set] + 31) / 32;
+    for (uint64_t base = static_cast<uint64_t>(blockIdx.x) * kThreads; base < words;
+         base += static_cast<uint64_t>(gridDim.x) * kThreads) {
+        const uint64_t w = base + threadIdx.x;
+        uint32_t word = 0;
+        if (w < words) {
+            word = s.changes[set][w] | s.stale[set][w];
+            const uint64_t tail = s.size[set] - w * 32;  // elements in this word
+            if (tail < 32) word &= (1u << tail) - 1u;
+        }
+        const uint32_t n = static_cast<uint32_t>(__popc(word));
+        const uint32_t incl = wave_incl_scan_u32(n);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, kWaveSize - 1);
+        if (total == 0) continue;  // wave-uniform
+        unsigned long long at = 0;
+        if (lane == 0) at = atomicAdd(&s.count[set], static_cast<unsigned long long>(total));
+        if (!s.list[set]) continue;
+        at = readlane_u64(at, 0) + incl - n;
+        while (word) {
+            const uint32_t bit = __ffs(word) - 1;
+            word &= word - 1;
+            s.list[set][at++] = static_cast<uint32_t>(w * 32 + bit);
+        }
+    }
+}
+
+// kTransposeRows listed rows per workgroup and turn through an LDS tile: whole
+// rows in, whole 128-byte runs of one output out.
+__global__ void __launch_bounds__(kThreads) leo_gather_rows(GatherRows g) {
+    __shared__ float tile[kTransposeRows][kOutputs];
+    for (uint64_t k0 = static_cast<uint64_t>(blockIdx.x) * kTransposeRows; k0 < g.count;
+         k0 += static_cast<uint64_t>(gridDim.x) * kTransposeRows) {
+        const uint32_t rows = static_cast<uint32_t>(g.count - k0 < kTransposeRows ? g.count - k0 : kTransposeRows);
+        for (uint32_t i = threadIdx.x; i < rows * kOutputs; i += kThreads) {
+            const uint32_t r = i / kOutputs, o = i % kOutputs;
+            tile[r][o] = g.rows[static_cast<uint64_t>(g.list[k0 + r]) * kOutStride + o];
+        }
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < kTransposeRows * kOutputs; i += kThreads) {
+            const uint32_t o = i / kTransposeRows, r = i % kTransposeRows;
+            if (r < rows) g.out[static_cast<uint64_t>(o) * g.count + k0 + r] = tile[r][o];
+        }
+        __syncthreads();
+    }
+}
+
+__global__ void __launch_bounds__(kThreads) leo_gather_slots(GatherSlots g) {
+    for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * kThreads + threadIdx.x; i < g.count * g.E;
+         i += static_cast<uint64_t>(gridDim.x) * kThreads) {
+        const uint64_t k = i / g.E, e = i - k * g.E, slot = g.list[k];
+        g.emb[i] = g.p.ctx_emb[slot * g.E + e];
+        if (e == 0) {
+            g.keys[k] = g.p.ctx_keys[slot];
+            g.obs[k] = g.p.ctx_obs[slot];
+        }
+    }
+}
+
 }  // namespace leo
