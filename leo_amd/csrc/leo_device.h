@@ -362,7 +362,7 @@ struct LaneDesc {
     const StepParams LEO_GLOBAL* steps;
     StepRecord LEO_GLOBAL* records;
     uint32_t step_count;
-    uint32_t pad;
+    uint32_t reset_tick;  // the lane's tick after a reset with kResetLaneTicks
     // where the launch's first thread stores the lane's outcome of the
     // previous launch (error code, error step, bias fail, tick) before this
     // launch can change it, for a host that reads the outcomes of a queue of
@@ -375,6 +375,10 @@ struct LaneDesc {
 };
 
 constexpr uint32_t kPhases = 8;
+
+// The tick a reset leaves: the lane's own, one for every lane, or each lane's
+// LaneDesc::reset_tick.
+enum : uint32_t { kResetKeepTick = 0, kResetTick = 1, kResetLaneTicks = 2 };
 
 // Read-only model data shared by every lane.
 struct SharedModel {

@@ -3930,7 +3930,7 @@ __global__ void __launch_bounds__(kThreads) leo_reset_lanes(KernelArgs args, uin
     // host has read the code and cleared it (a reset queued behind the
     // failing launch does nothing)
     if (d.ctl->error_code != 0) return;
-    const uint32_t tick = set_tick ? new_tick : d.ctl->tick;
+    const uint32_t tick = set_tick == kResetKeepTick ? d.ctl->tick : set_tick == kResetTick ? new_tick : d.reset_tick;
     const uint64_t N = cfg.neuron_count, S = cfg.synapses_per_neuron;
     const uint64_t NS = N * S, NI = static_cast<uint64_t>(kSymbols) * cfg.input_fanout;
     const uint64_t t0 = static_cast<uint64_t>(part) * kThreads + threadIdx.x, ts = static_cast<uint64_t>(parts) * kThreads;
