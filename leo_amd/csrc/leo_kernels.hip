@@ -3262,65 +3262,79 @@ __device__ __forceinline__ float inhibitory_step(const LeoConfig& cfg, float w, 
     return clampf(w + delta, cfg.weight_min, 0.0f);
 }
 
+// The context projection and embeddings (runtime.rs:1318-1384), on the readout
+// workgroup, which holds the step's cells, scales and latent in LDS. Sixteen
+// dimensions of the projection at a time: one round of loads, kept in
+// registers for the update and in LDS for the embeddings' gradient, whose sums
+// are serial in output order, one dimension a thread. The embeddings and
+// counts it will update are loaded in the same round. With the projection
+// loaded twice, 32 outputs of a dimension at a time, and a division for every
+// element's place, this held the learning phase for ~8 us a step; a document at
+// 16,384 units took 7.38 ms of step kernel then and 7.26 now (other workgroups
+// of the phase are nearly as long).
 __device__ __forceinline__ void context_update(const StepCtx& c, const StepParams& sp, StepShared& sh,
                                                uint32_t step_index) {
     const LeoConfig& cfg = c.a->cfg;
     const LaneDesc& d = c.d;
     LaneControl* ctl = c.ctl;
-    const uint32_t E = cfg.context_embedding_dim, count = ld(&ctl->ctx_count);
+    const uint32_t E = cfg.context_embedding_dim, count = sh.ctx_cells;
     const float lr = cfg.context_learning_rate, mu = cfg.max_update, wmin = cfg.weight_min, wmax = cfg.weight_max;
     const float strength = sp.supervised_strength;
-    float* grad = sh.aux;
-    // serial in output order; the weights of 32 outputs are loaded at a time
-    constexpr uint32_t kChunk = 32;
-    for (uint32_t e = threadIdx.x; e < E; e += kThreads) {
-        float g = 0.0f;
-        for (uint32_t o0 = 0; o0 < kOutputs; o0 += kChunk) {
-            float w[kChunk];
-#pragma unroll
-            for (uint32_t k = 0; k < kChunk; ++k) w[k] = o0 + k < kOutputs ? ld(&d.p.ctx_out[(o0 + k) * E + e]) : 0.0f;
-#pragma unroll
-            for (uint32_t k = 0; k < kChunk; ++k)
-                if (o0 + k < kOutputs) g += w[k] * sh.err[o0 + k];
-        }
-        grad[e] = g;
-    }
-    __syncthreads();
+    constexpr uint32_t kDims = 16, kEach = (kOutputs * kDims + kThreads - 1) / kThreads;
+    float* tile = reinterpret_cast<float*>(step_lds);  // kOutputs * kDims
+    float* grad = sh.aux;                              // kMaxEmbedding
+    static_assert(kMaxEmbedding <= kOutStride + kThreads, "the gradient fits");
+    const uint32_t cells = count * E;
+    const uint32_t cell0 = threadIdx.x < cells ? threadIdx.x / E : 0u;
+    const uint64_t emb0 = threadIdx.x < cells
+                              ? static_cast<uint64_t>(sh.ctx_cell[cell0]) * E + (threadIdx.x - cell0 * E) : 0u;
+    const float old0 = threadIdx.x < cells ? ld(&d.p.ctx_emb[emb0]) : 0.0f;
+    const uint32_t obs = threadIdx.x < count ? ld(&d.p.ctx_obs[sh.ctx_cell[threadIdx.x]]) : 0u;
     if (threadIdx.x == 0) ctl->ctx_out_dirty = 1;
-    // four elements per thread at a time, their loads together
-    constexpr uint32_t kBatch = 4;
-    for (uint32_t i0 = threadIdx.x; i0 < kOutputs * E; i0 += kBatch * kThreads) {
-        float old[kBatch], latent[kBatch];
+    for (uint32_t e0 = 0; e0 < E; e0 += kDims) {
+        float w[kEach];
 #pragma unroll
-        for (uint32_t k = 0; k < kBatch; ++k) {
-            const uint32_t i = i0 + k * kThreads;
-            old[k] = i < kOutputs * E ? ld(&d.p.ctx_out[i]) : 0.0f;
-            latent[k] = i < kOutputs * E ? ld(&d.ctx_latent[i % E]) : 0.0f;
+        for (uint32_t k = 0; k < kEach; ++k) {
+            const uint32_t i = threadIdx.x + k * kThreads, o = i / kDims, e = e0 + i % kDims;
+            w[k] = o < kOutputs && e < E ? ld(&d.p.ctx_out[o * E + e]) : 0.0f;
         }
 #pragma unroll
-        for (uint32_t k = 0; k < kBatch; ++k) {
-            const uint32_t i = i0 + k * kThreads;
-            if (i >= kOutputs * E) continue;
-            const float gradient = sh.err[i / E] * latent[k];
+        for (uint32_t k = 0; k < kEach; ++k) {
+            const uint32_t i = threadIdx.x + k * kThreads;
+            if (i < kOutputs * kDims) tile[i] = w[k];
+        }
+        __syncthreads();
+        if (threadIdx.x < kDims && e0 + threadIdx.x < E) {
+            float g = 0.0f;
+#pragma unroll 16
+            for (uint32_t o = 0; o < kOutputs; ++o) g += tile[o * kDims + threadIdx.x] * sh.err[o];
+            grad[e0 + threadIdx.x] = g;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kEach; ++k) {
+            const uint32_t i = threadIdx.x + k * kThreads, o = i / kDims, e = e0 + i % kDims;
+            if (o >= kOutputs || e >= E) continue;
+            const float gradient = sh.err[o] * sh.latent[e];
             const float delta = bounded(-lr * strength * gradient, mu);
-            const float updated = clampf(old[k] + delta, wmin, wmax);
+            const float updated = clampf(w[k] + delta, wmin, wmax);
             if (!finitef(updated)) set_step_error(ctl, kErrContextProjection, step_index);
-            d.p.ctx_out[i] = updated;
+            d.p.ctx_out[o * E + e] = updated;
         }
+        __syncthreads();
     }
-    for (uint32_t i = threadIdx.x; i < count * E; i += kThreads) {
-        const uint32_t k = i / E, e = i % E;
-        const uint64_t slot = ld(&ctl->ctx_slots[k]);
-        const float gradient = ld(&ctl->ctx_scales[k]) * grad[e];
+    for (uint32_t i = threadIdx.x; i < cells; i += kThreads) {
+        const uint32_t k = i / E, e = i - k * E;
+        const uint64_t at = static_cast<uint64_t>(sh.ctx_cell[k]) * E + e;
+        const float old = i == threadIdx.x ? old0 : ld(&d.p.ctx_emb[at]);
+        const float gradient = sh.ctx_weight[k] * grad[e];
         const float delta = bounded(-lr * strength * gradient, mu);
-        const float updated = clampf(ld(&d.p.ctx_emb[slot * E + e]) + delta, wmin, wmax);
+        const float updated = clampf(old + delta, wmin, wmax);
         if (!finitef(updated)) set_step_error(ctl, kErrContextEmbedding, step_index);
-        d.p.ctx_emb[slot * E + e] = updated;
+        d.p.ctx_emb[at] = updated;
     }
-    for (uint32_t k = threadIdx.x; k < count; k += kThreads) {
-        const uint32_t slot = ld(&ctl->ctx_slots[k]);
+    if (threadIdx.x < count) {
+        const uint32_t slot = sh.ctx_cell[threadIdx.x];
         mark_bit(d.ch_ctx, slot);
-        const uint32_t obs = ld(&d.p.ctx_obs[slot]);
         d.p.ctx_obs[slot] = obs == 0xffffffffu ? obs : obs + 1;
     }
     __syncthreads();
@@ -3387,7 +3401,7 @@ __device__ __forceinline__ void phase_learn(const StepCtx& c, const StepParams& 
                 ctl->bias_dirty = 1;
                 if (bias_fail != kNoFail) set_step_error(ctl, kErrBias, step_index);
             }
-            if (bias_fail == kNoFail && ld(&ctl->ctx_applied) && ld(&ctl->ctx_count) > 0)
+            if (bias_fail == kNoFail && sh.ctx_cells > 0)  // no cells without an applied context
                 context_update(c, sp, sh, step_index);
         }
         if (plastic && bias_fail == kNoFail) {
