@@ -2858,10 +2858,11 @@ __device__ __forceinline__ void context_logits(const StepCtx& c, StepShared& sh)
 
 // The readout's list of active neurons, from the selecting waves' winners (the
 // active list of a non-binding cap, still being written in this phase): the
-// ids and activations of list places [b0, b0 + kThreads) into LDS, one thread
-// per selecting wave, its first winner loaded with its total. Returns the
-// list's length.
-__device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& sh, uint32_t b0, uint32_t* ids, float* acts) {
+// ids and activations into LDS, one thread per selecting wave, its first winner
+// loaded with its total. Returns the list's length; a list longer than kThreads
+// is not listed (a thread would walk thousands of winners one by one: the
+// readout then searches each place's wave instead).
+__device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& sh, uint32_t* ids, float* acts) {
     const LaneDesc& d = c.d;
     const LeoConfig& cfg = c.a->cfg;
     const uint32_t nwaves = selecting_waves(c), wave = wave_index(), lane = __lane_id();
@@ -2884,9 +2885,8 @@ __device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& s
             at += w < wave ? total : 0u;
             running += total;
         }
-        for (uint32_t i = 0; i < count; ++i) {
-            const uint32_t f = at + i - b0;  // wraps past kThreads below b0
-            if (f >= kThreads) continue;
+        for (uint32_t i = 0; running <= kThreads && i < count; ++i) {
+            const uint32_t f = at + i;
             ids[f] = i == 0 ? n0 : ld(&d.range_winners[row0 + i]);
             acts[f] = i == 0 ? act0 : ld(&d.range_winner_act[row0 + i]);
         }
@@ -2923,6 +2923,8 @@ __device__ __forceinline__ uint32_t readout(const StepCtx& c, const StepParams& 
     uint32_t* ids = reinterpret_cast<uint32_t*>(step_lds);
     float* acts = reinterpret_cast<float*>(step_lds) + kThreads;
     float* ends = reinterpret_cast<float*>(step_lds) + 2 * kThreads;
+    uint32_t* starts = reinterpret_cast<uint32_t*>(step_lds) + 3 * kThreads;  // a list longer than kThreads
+    const uint32_t nwaves = selecting_waves(c), range = (cfg.block_count + nwaves - 1) / nwaves;
     StepRecord LEO_GLOBAL& rec = d.records[step_index];
     if (end_thread) {
         rec.p_target = 0.0f;
@@ -2948,7 +2950,21 @@ __device__ __forceinline__ uint32_t readout(const StepCtx& c, const StepParams& 
         ids[threadIdx.x] = 0u;
         __syncthreads();
         if (from_waves) {
-            A = list_winners(c, sh, b0, ids, acts);
+            if (b0 == 0) {
+                A = list_winners(c, sh, ids, acts);
+                if (A > kThreads) wave_starts(c, sh, starts, nwaves);
+            }
+            if (A > kThreads) {
+                uint32_t n = 0;
+                float act = 0.0f;
+                if (b0 + threadIdx.x < A) {
+                    (void)winner_key(d, starts, nwaves, range, cfg.block_count, cfg.max_active_per_block,
+                                     b0 + threadIdx.x, cfg.neuron_count, 0u, &n, &act);
+                    ids[threadIdx.x] = n;
+                    acts[threadIdx.x] = act;
+                }
+                __syncthreads();
+            }
         } else if (b0 + threadIdx.x < A) {
             const uint64_t at = static_cast<uint64_t>(rs) * cfg.max_active_global + b0 + threadIdx.x;
             ids[threadIdx.x] = ld(&d.ring_active[at]);
