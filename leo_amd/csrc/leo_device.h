@@ -58,8 +58,9 @@ constexpr uint32_t kFixedEntries = 4;
 inline __host__ __device__ uint32_t window_capacity(uint32_t neurons_per_block) {
     return neurons_per_block > 256 ? neurons_per_block : 256;
 }
-// Per-wave bytes of the window: touched neurons, then the candidates' u64 keys,
-// blocks and order by block (capacity each), and the group's block starts.
+// Per-wave bytes of the window: the candidates' u64 keys, the touched neurons
+// or the keys by block, both orders' blocks (capacity each), and the group's
+// block starts.
 inline __host__ __device__ size_t window_bytes(uint32_t neurons_per_block) {
     const size_t c = window_capacity(neurons_per_block);
     return (c * 20 + (kGroupBlocks + 1) * 4 + 15) / 16 * 16;

@@ -1255,9 +1255,9 @@ struct DeepArray {
 constexpr uint32_t kDeepTiles = 8;  // 64-entry tiles a lane has in flight
 
 // The ranks of K entries per lane among `cnt` keys in LDS (distinct, padded to
-// a multiple of four with the largest key): the number of smaller keys. Four
-// keys per 16-byte LDS read (the same address on every lane), two instructions
-// per key and entry.
+// a multiple of four with the largest key): the number of smaller keys. Words
+// four per 16-byte LDS read, wider keys two (the same address on every lane),
+// two instructions per key and entry.
 template <uint32_t K, class Key>
 __device__ __forceinline__ void deep_ranks(const Key* keys, uint32_t cnt, const Key (&mine)[4], uint32_t (&rank)[4]) {
     for (uint32_t q = 0; q < cnt; q += 4) {
@@ -1560,13 +1560,15 @@ __device__ __forceinline__ float surrogate_value(const LeoConfig& cfg, bool refr
 // Phase-2 window of one wave in dynamic LDS (window_bytes per wave): the
 // touched neurons of a run of blocks in any order, and those of them above
 // threshold (the candidates) with their selection keys and blocks. More than
-// 64 candidates are also sorted by block (`order`, `first`).
+// kPairwise candidates of several blocks are also sorted by block (`sorted`,
+// `sorted_block`, `first`).
 struct Window {
-    uint64_t* key;     // capacity: a candidate's selection key
-    uint32_t* entry;   // capacity: a touched neuron
-    uint32_t* block;   // capacity: a candidate's block, counted from the group's first
-    uint32_t* order;   // capacity: candidates by block
-    uint32_t* first;   // kGroupBlocks + 1: each block's first place in `order`
+    uint64_t* key;           // capacity: a candidate's selection key
+    uint32_t* entry;         // capacity: a touched neuron (in the place of `sorted`, which is written after the folds)
+    uint64_t* sorted;        // capacity: the keys by block
+    uint16_t* block;         // capacity: a candidate's block, counted from the group's first
+    uint16_t* sorted_block;  // capacity: the sorted keys' blocks
+    uint32_t* first;         // kGroupBlocks + 1: each block's first place in `sorted`
 };
 
 static_assert(kGroupBlocks == kWaveSize, "one lane per group block");
@@ -1576,10 +1578,11 @@ __device__ __forceinline__ Window wave_window(uint32_t wave, uint32_t nb) {
     const uint32_t cap = window_capacity(nb);
     Window w;
     w.key = reinterpret_cast<uint64_t*>(base);
-    w.entry = reinterpret_cast<uint32_t*>(w.key + cap);
-    w.block = w.entry + cap;
-    w.order = w.block + cap;
-    w.first = w.order + cap;
+    w.sorted = w.key + cap;
+    w.entry = reinterpret_cast<uint32_t*>(w.sorted);
+    w.block = reinterpret_cast<uint16_t*>(w.sorted + cap);
+    w.sorted_block = w.block + cap;
+    w.first = reinterpret_cast<uint32_t*>(w.sorted_block + cap);
     return w;
 }
 
@@ -1590,8 +1593,11 @@ struct Placed {
     uint32_t rank, before;
 };
 
-// Up to 64 candidates, one a lane: every pair through lane reads (a sparse
-// tick leaves a wave a few candidates). Every lane of the wave calls.
+// Up to kPairwise candidates, one a lane: every pair through lane reads (a
+// sparse tick leaves a wave a few candidates). Every lane of the wave calls.
+// Frozen steps with 16, 32 and 64 as the limit: 20 to 60 candidates of ~6
+// blocks a wave 16.2, 16.7 and 17.7 us, ~31 of one block 11.3, 11.4 and 12.2.
+constexpr uint32_t kPairwise = 16;
 __device__ __forceinline__ Placed place_few(uint64_t key, uint32_t block, uint32_t nc, uint32_t limit) {
     Placed p{0, 0};
     for (uint32_t q = 0; q < nc; ++q) {
@@ -1608,9 +1614,9 @@ __device__ __forceinline__ Placed place_few(uint64_t key, uint32_t block, uint32
     return p;
 }
 
-// More than 64 candidates: sorted by block first (counts, a scan, places), so
-// that each is compared with its own block's candidates only. Leaves the
-// blocks' winner positions in `base` lanes (lane g: block g of the group).
+// More candidates of several blocks: their keys sorted by block (counts, a
+// scan, places), so that each is compared with its own block's keys only.
+// Returns the blocks' winner positions (lane g: block g of the group).
 __device__ __forceinline__ uint32_t sort_by_block(const Window& w, uint32_t nc, uint32_t limit) {
     const uint32_t lane = __lane_id();
     w.first[lane] = 0u;
@@ -1622,12 +1628,32 @@ __device__ __forceinline__ uint32_t sort_by_block(const Window& w, uint32_t nc, 
     wave_sync();
     w.first[lane] = start;
     wave_sync();
-    for (uint32_t i = lane; i < nc; i += kWaveSize) w.order[atomicAdd(&w.first[w.block[i]], 1u)] = i;
+    for (uint32_t i = lane; i < nc; i += kWaveSize) {
+        const uint16_t block = w.block[i];
+        const uint32_t at = atomicAdd(&w.first[block], 1u);
+        w.sorted[at] = w.key[i];
+        w.sorted_block[at] = block;
+    }
     wave_sync();
     w.first[lane] = start;
     if (lane == 0) w.first[kGroupBlocks] = nc;
     wave_sync();
     return wave_incl_scan_u32(won) - won;
+}
+
+// The number of keys[j, j1) smaller than `key`. Eight independent LDS reads a
+// round: one read at a time waits out the LDS latency on every key.
+__device__ __forceinline__ uint32_t count_smaller(const uint64_t* keys, uint32_t j, uint32_t j1, uint64_t key) {
+    uint32_t smaller = 0;
+    for (; j + 8 <= j1; j += 8) {
+        uint64_t k[8];
+#pragma unroll
+        for (uint32_t x = 0; x < 8; ++x) k[x] = keys[j + x];
+#pragma unroll
+        for (uint32_t x = 0; x < 8; ++x) smaller += k[x] < key ? 1u : 0u;
+    }
+    for (; j < j1; ++j) smaller += keys[j] < key ? 1u : 0u;
+    return smaller;
 }
 
 // Phase 2: each wave owns a range of blocks and takes it in groups of up to
@@ -1641,6 +1667,13 @@ __device__ __forceinline__ uint32_t sort_by_block(const Window& w, uint32_t nc, 
 // staged in block order (runtime.rs:1010-1013), compacted from the range's
 // first block row, so that phase 3 reads them in one round. A group with more
 // touched neurons than the window holds is taken in runs of whole blocks.
+// More than kPairwise candidates are compared through independent LDS reads:
+// those of one block four own keys a lane against four broadcast keys a read
+// (deep_ranks), those of several blocks sorted first and eight keys a round
+// (count_smaller). Frozen steps with ~230 candidates in a wave's one block of
+// 256 took 91 us when each comparison was a dependent pair of LDS reads, 37
+// with eight keys a round after listing in neuron order, and take 29; with
+// ~910 in a block of 1,024 they took 1,015, 268 and take 182.
 // Bound by the chain of dependent instructions and memory rounds of one wave
 // per SIMD, not by bandwidth. Listing in neuron order took a scan and LDS
 // writes per row of 64 words, and block starts, counts and ranks went through
@@ -1800,22 +1833,43 @@ __device__ __forceinline__ void phase_fold_select(const StepCtx& c, StepShared& 
                 }
             }
             wave_sync();
-            if (nc <= kWaveSize) {
+            if (nc <= kPairwise) {
                 const uint64_t key = lane < nc ? w.key[lane] : ~0ULL;
                 const uint32_t block = lane < nc ? w.block[lane] : ~0u;
                 const Placed at = place_few(key, block, nc, limit);
                 if (lane < nc) place(key, gb + block, at);
                 staged += static_cast<uint32_t>(__popcll(__ballot(lane < nc && at.rank < limit)));
+            } else if (e - s == 1) {
+                // one block: its keys as they are, padded to whole quarters,
+                // four of the wave's own candidates a lane at a time
+                const uint32_t padded = (nc + 3) & ~3u;
+                if (nc + lane < padded) w.key[nc + lane] = ~0ULL;
+                wave_sync();
+                for (uint32_t i0 = 0; i0 < nc; i0 += 4 * kWaveSize) {
+                    uint64_t key[4];
+                    uint32_t rank[4] = {0, 0, 0, 0};
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        const uint32_t i = i0 + k * kWaveSize + lane;
+                        key[k] = i < nc ? w.key[i] : ~0ULL;
+                    }
+                    if (nc - i0 <= kWaveSize) deep_ranks<1>(w.key, nc, key, rank);
+                    else if (nc - i0 <= 2 * kWaveSize) deep_ranks<2>(w.key, nc, key, rank);
+                    else deep_ranks<4>(w.key, nc, key, rank);
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k)
+                        if (i0 + k * kWaveSize + lane < nc) place(key[k], gb + s, Placed{rank[k], 0});
+                }
+                staged += min(nc, limit);
             } else {
                 const uint32_t base = sort_by_block(w, nc, limit);
                 uint32_t won = 0;
                 for (uint32_t i0 = 0; i0 < nc; i0 += kWaveSize) {
                     const uint32_t i = i0 + lane;
-                    const uint64_t key = i < nc ? w.key[i] : ~0ULL;
-                    const uint32_t block = i < nc ? w.block[i] : 0u;
+                    const uint64_t key = i < nc ? w.sorted[i] : ~0ULL;
+                    const uint32_t block = i < nc ? w.sorted_block[i] : 0u;
                     Placed at{0, static_cast<uint32_t>(__shfl(static_cast<int>(base), static_cast<int>(block)))};
-                    const uint32_t j1 = i < nc ? w.first[block + 1] : 0u;
-                    for (uint32_t j = w.first[block]; j < j1; ++j) at.rank += w.key[w.order[j]] < key ? 1u : 0u;
+                    at.rank = count_smaller(w.sorted, w.first[block], i < nc ? w.first[block + 1] : 0u, key);
                     if (i < nc) place(key, gb + block, at);
                     won += static_cast<uint32_t>(__popcll(__ballot(i < nc && at.rank < limit)));
                 }

@@ -1,0 +1,68 @@
+"""Kernel time of dense steps against sparse ones of the same model in the same
+process: what a step does per candidate has to stay a small part of it. The
+limits lie between the time ratios measured with a batched and with a serial
+form of the work (both stated), near their geometric mean."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from leo_amd import native
+from leo_amd.config import Config
+from leo_amd.config import test_toml_values as toml_values
+from leo_amd.model import Model
+from tests.helpers import story
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(nb, blocks, fanout, limit, strength=1.0):
+    """Input edges strong enough (at 1.0) that most injected neurons are above their threshold."""
+    values = toml_values()
+    n = nb * blocks
+    values["model"].update(neuron_count=n, block_count=blocks, neurons_per_block=nb, synapses_per_neuron=6,
+                           input_fanout=fanout, max_active_per_block=limit, max_active_global=blocks * limit)
+    values["dynamics"].update(target_activity=min(0.5, 0.9 * limit / nb), population_inhibition_rate=0.001)
+    model = Model.synthetic(Config.from_dict(values), weight_sigma=0.05)
+    rng = np.random.default_rng(nb * 1000 + fanout)
+    model.in_target.reshape(258, fanout)[:] = [rng.permutation(n)[:fanout] for _ in range(258)]
+    model.in_branch[:] = 0
+    model.in_weight[:] = (strength * rng.uniform(0.3, 1.0, model.in_weight.size)).astype(np.float32)
+    model.threshold[:] = np.float32(0.4)
+    model.validate()
+    return model
+
+
+def _step_us(model, run, steps):
+    """Best kernel time per step of five passes."""
+    from leo_amd.runtime import HipRuntime
+
+    gpu = HipRuntime(model, device=0, max_lanes=1)
+    try:
+        best = float("inf")
+        for _ in range(5):
+            gpu.kernel_stats(reset=True)
+            run(gpu)
+            best = min(best, gpu.kernel_stats()["kernel_ms"] * 1e3 / steps)
+        return best
+    finally:
+        gpu.close()
+
+
+TEXT = story(5, 120)
+
+
+def _frozen(gpu):
+    gpu.begin_document()
+    gpu.advance_frozen_batch([(b, None) for b in TEXT])
+
+
+# Frozen steps with nearly every neuron of a wave's one block a candidate,
+# against the same deliveries with none. With one dependent pair of LDS reads a
+# comparison 46 and 7.5 times; with independent reads 8.4 and 2.4.
+@pytest.mark.parametrize("nb,blocks,fanout,limit,most", [(1024, 2, 1900, 64, 20.0), (256, 4, 1000, 16, 4.2)])
+def test_ranking_many_candidates(require_gpu, nb, blocks, fanout, limit, most):
+    none = _step_us(_model(nb, blocks, fanout, limit, 0.001), _frozen, len(TEXT))
+    dense = _step_us(_model(nb, blocks, fanout, limit), _frozen, len(TEXT))
+    print(f"{blocks} blocks of {nb}: {none:.1f} us a step without candidates, {dense:.1f} us with", flush=True)
+    assert dense < most * none

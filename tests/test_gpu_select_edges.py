@@ -1,6 +1,7 @@
 """Block selection at the edges of a wave's window against the oracle: touched
 neurons below and past its 256 entries, few candidates (placed through lane
-reads) and more than 64 (sorted by block), blocks smaller than a bitmap word,
+reads) and more (one block's compared as they are, several blocks' sorted
+first), blocks smaller than a bitmap word,
 not a multiple of one, and of the largest size. Inputs strong enough that most
 injected neurons are candidates; losses, lists and the model bit for bit."""
 from __future__ import annotations
@@ -19,6 +20,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # neurons per block, blocks, input edges per symbol, winners per block
     (16, 64, 40, 2), (16, 640, 900, 3), (20, 96, 500, 5), (96, 40, 63, 4), (96, 40, 1500, 90),
     (200, 24, 65, 8), (256, 4, 64, 8), (256, 4, 700, 16), (256, 520, 4000, 1), (1024, 2, 1900, 64),
+    (256, 4, 160, 16), (64, 64, 1300, 16),
 ]
 
 
