@@ -1741,35 +1741,55 @@ __device__ __forceinline__ void phase_fold_select(const StepCtx& c, StepShared& 
         // loads past them return 0, so that no lane is masked
         const __amdgpu_buffer_rsrc_t bits =
             coherent_rsrc(set_touched(d, set) + static_cast<uint64_t>(gb) * wpb, gw * 4);
+        // of a group that the window does not hold: the touched neurons of
+        // blocks 0..lane, which give every run's end after one scan (kept
+        // instead of the words, whose registers the folds need: each run loads
+        // its own again). With all of the group's words loaded again and the
+        // end searched by halving from the group's, a frozen step of four
+        // waves with 2,000 to 3,000 touched neurons each took 195 us (64
+        // blocks a wave) and 289 us (16), and takes 178 and 277.
+        bool full = false;
+        uint32_t ends = 0;
         for (uint32_t s = 0; s < gn;) {
             // the run of blocks [s, e): the rest of the group, or as many of
-            // its blocks as the window is sure to hold (a block holds at most
-            // nb <= cap); the words are loaded again for each run rather than
-            // kept in registers through the folds (a sparse tick has one run)
+            // its blocks as the window holds (a block holds at most nb <= cap)
+            uint32_t e = gn;
+            auto run_end = [&] {
+                const uint32_t before = s > 0 ? __builtin_amdgcn_readlane(ends, static_cast<int>(s - 1)) : 0u;
+                const uint64_t fits = __ballot(lane < gn && ends - before <= cap);  // (blocks before s wrap around)
+                return max(s + 1, s + static_cast<uint32_t>(__popcll(fits >> s)));
+            };
+            if (__builtin_expect(full, 0)) e = run_end();
             uint32_t word[kWordsPerLane];
 #pragma unroll
             for (uint32_t k = 0; k < kWordsPerLane; ++k) {
+                const uint32_t at = s * wpb + k * kWaveSize;
                 word[k] = 0u;
-                if (k * kWaveSize < gw)
-                    word[k] = __builtin_amdgcn_raw_buffer_load_b32(bits, (k * kWaveSize + lane) * 4, 0, 16);
+                if (at < e * wpb) word[k] = __builtin_amdgcn_raw_buffer_load_b32(bits, (at + lane) * 4, 0, 16);
             }
-            if (s > 0) {
-#pragma unroll
-                for (uint32_t k = 0; k < kWordsPerLane; ++k)
-                    if (k * kWaveSize + lane < s * wpb) word[k] = 0u;
-            }
-            uint32_t e = gn, incl = 0, total = 0;
-            for (;;) {
+            uint32_t incl = 0, total = 0;
+            auto scan = [&] {
                 uint32_t part = 0;
 #pragma unroll
-                for (uint32_t k = 0; k < kWordsPerLane; ++k) part += __popc(word[k]);
+                for (uint32_t k = 0; k < kWordsPerLane; ++k) {
+                    if (s * wpb + k * kWaveSize + lane >= e * wpb) word[k] = 0u;
+                    part += __popc(word[k]);
+                }
                 incl = wave_incl_scan_u32(part);
                 total = __builtin_amdgcn_readlane(incl, kWaveSize - 1);
-                if (__builtin_expect(total <= cap, 1) || e == s + 1) break;
-                e = s + (e - s + 1) / 2;
+            };
+            scan();
+            if (__builtin_expect(total > cap, 0)) {  // the group's first run
+                full = true;
+                w.first[lane] = 0u;
+                wave_sync();
 #pragma unroll
                 for (uint32_t k = 0; k < kWordsPerLane; ++k)
-                    if (k * kWaveSize + lane >= e * wpb) word[k] = 0u;
+                    if (word[k]) atomicAdd(&w.first[fast_div(k * kWaveSize + lane, block_div)], __popc(word[k]));
+                wave_sync();
+                ends = wave_incl_scan_u32(w.first[lane]);
+                e = run_end();
+                scan();
             }
             // the words are cleared after all have arrived: a store issued
             // between the loads would be waited for together with the later
@@ -1778,15 +1798,16 @@ __device__ __forceinline__ void phase_fold_select(const StepCtx& c, StepShared& 
             if (!keep_bits) {
 #pragma unroll
                 for (uint32_t k = 0; k < kWordsPerLane; ++k) {
-                    if (word[k]) __builtin_amdgcn_raw_buffer_store_b32(0u, bits, (k * kWaveSize + lane) * 4, 0, 0);
+                    if (word[k])
+                        __builtin_amdgcn_raw_buffer_store_b32(0u, bits, (s * wpb + k * kWaveSize + lane) * 4, 0, 0);
                 }
             }
             uint32_t p = incl;  // this lane's neurons end here
 #pragma unroll
             for (uint32_t k = 0; k < kWordsPerLane; ++k) {
                 uint32_t v = word[k];
-                if (k * kWaveSize < gw && v != 0) {
-                    const uint32_t at = k * kWaveSize + lane, g = fast_div(at, block_div);
+                if (s * wpb + k * kWaveSize < e * wpb && v != 0) {
+                    const uint32_t at = s * wpb + k * kWaveSize + lane, g = fast_div(at, block_div);
                     const uint32_t n0 = (gb + g) * nb + (at - g * wpb) * 32;
                     do {
                         w.entry[--p] = n0 + __ffs(v) - 1;

@@ -24,6 +24,18 @@ SHAPES = [  # neurons per block, blocks, input edges per symbol, winners per blo
 ]
 
 
+RUNS = [  # one workgroup's four waves: groups of 64 blocks (40 of 320 neurons) in runs of many, few and one block
+    (16, 260, 2200, 3), (64, 256, 3000, 4), (256, 66, 2400, 4), (256, 16, 3900, 8), (320, 48, 2500, 5),
+]
+
+
+@pytest.mark.parametrize("nb,blocks,fanout,limit", RUNS)
+def test_runs_of_blocks_match_oracle(require_gpu, oracle, monkeypatch, nb, blocks, fanout, limit):
+    monkeypatch.setenv("LEO_HIP_WGS_PER_LANE", "1")
+    monkeypatch.setenv("LEO_HIP_CANONICAL_WGS", "1")
+    test_selection_matches_oracle(require_gpu, oracle, nb, blocks, fanout, limit)
+
+
 @pytest.mark.parametrize("nb,blocks,fanout,limit", SHAPES)
 def test_selection_matches_oracle(require_gpu, oracle, nb, blocks, fanout, limit):
     from leo_amd.runtime import HipRuntime
