@@ -193,14 +193,20 @@ __device__ __forceinline__ uint32_t dpp_keep_u32(uint32_t x) {
         __builtin_amdgcn_update_dpp(static_cast<int>(x), static_cast<int>(x), kCtrl, kRowMask, 0xf, false));
 }
 template <class Max>
-__device__ __forceinline__ uint32_t wave_reduce_max(uint32_t v, Max&& larger) {
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v, Max&& larger) {  // lane i: of lanes 0..i
     v = larger(v, dpp_keep_u32<0x111, 0xf>(v));
     v = larger(v, dpp_keep_u32<0x112, 0xf>(v));
     v = larger(v, dpp_keep_u32<0x114, 0xf>(v));
     v = larger(v, dpp_keep_u32<0x118, 0xf>(v));
     v = larger(v, dpp_keep_u32<0x142, 0xa>(v));
-    v = larger(v, dpp_keep_u32<0x143, 0xc>(v));
-    return __builtin_amdgcn_readlane(v, kWaveSize - 1);
+    return larger(v, dpp_keep_u32<0x143, 0xc>(v));
+}
+template <class Max>
+__device__ __forceinline__ uint32_t wave_reduce_max(uint32_t v, Max&& larger) {
+    return __builtin_amdgcn_readlane(wave_incl_max(v, larger), kWaveSize - 1);
+}
+__device__ __forceinline__ uint32_t wave_incl_max_u32(uint32_t v) {
+    return wave_incl_max(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
 }
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return wave_reduce_max(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
@@ -2932,17 +2938,25 @@ __device__ __forceinline__ void context_logits(const StepCtx& c, StepShared& sh)
 }
 
 // The readout's list of active neurons, from the selecting waves' winners (the
-// active list of a non-binding cap, still being written in this phase): the
-// ids and activations into LDS, one thread per selecting wave, its first winner
-// loaded with its total. Returns the list's length; a list longer than kThreads
-// is not listed (a thread would walk thousands of winners one by one: the
-// readout then searches each place's wave instead).
-__device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& sh, uint32_t* ids, float* acts) {
+// active list of a non-binding cap, still being written in this phase), 256
+// places at a time.
+struct WinnerList {
+    uint32_t* ids;     // kThreads places
+    float* acts;       // kThreads places
+    uint32_t* owner;   // kThreads places: a wave + 1 at its first place here, else 0
+    uint32_t* starts;  // each selecting wave's first place, then the list's length
+};
+
+// The waves' first places, and the first 256 places as far as they are waves'
+// first winners, which are loaded beside the totals: a sparse tick's list
+// takes one memory round. One thread per selecting wave; `owner` is clear.
+// Returns the list's length; `more`: some wave has further winners.
+__device__ __forceinline__ uint32_t list_first_winners(const StepCtx& c, StepShared& sh, const WinnerList& l, bool* more) {
     const LaneDesc& d = c.d;
     const LeoConfig& cfg = c.a->cfg;
     const uint32_t nwaves = selecting_waves(c), wave = wave_index(), lane = __lane_id();
     const uint32_t range = (cfg.block_count + nwaves - 1) / nwaves;
-    uint32_t running = 0;
+    uint32_t running = 0, further = 0;
     for (uint32_t base = 0; base < nwaves; base += kThreads) {
         const uint32_t wv = base + threadIdx.x;
         const bool owns = wv < nwaves && wv * range < cfg.block_count;
@@ -2951,7 +2965,11 @@ __device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& s
         const uint32_t n0 = owns ? ld(&d.range_winners[row0]) : 0u;
         const float act0 = owns ? ld(&d.range_winner_act[row0]) : 0.0f;
         const uint32_t incl = wave_incl_scan_u32(count);
-        if (lane == kWaveSize - 1) sh.red[0][wave] = incl;
+        const uint64_t several = __ballot(count > 1);
+        if (lane == kWaveSize - 1) {
+            sh.red[0][wave] = incl;
+            sh.red[1][wave] = several ? 1u : 0u;
+        }
         __syncthreads();
         uint32_t at = running + incl - count;
 #pragma unroll
@@ -2959,15 +2977,56 @@ __device__ __forceinline__ uint32_t list_winners(const StepCtx& c, StepShared& s
             const uint32_t total = sh.red[0][w];
             at += w < wave ? total : 0u;
             running += total;
+            further |= sh.red[1][w];
         }
-        for (uint32_t i = 0; running <= kThreads && i < count; ++i) {
-            const uint32_t f = at + i;
-            ids[f] = i == 0 ? n0 : ld(&d.range_winners[row0 + i]);
-            acts[f] = i == 0 ? act0 : ld(&d.range_winner_act[row0 + i]);
+        if (wv < nwaves) l.starts[wv] = at;
+        if (count > 0 && at < kThreads) {
+            l.ids[at] = n0;
+            l.acts[at] = act0;
+            l.owner[at] = wv + 1;
         }
         __syncthreads();
     }
+    if (threadIdx.x == 0) l.starts[nwaves] = running;
+    *more = further != 0;
     return running;
+}
+
+// Places b0.. of the list of A winners, one thread a place: its wave is the
+// last one with a first place up to here (a maximum scan over `owner`; waves
+// without winners have none), and one memory round brings every winner that
+// is not there yet. The readout of 128 winners in each of two waves took 46.9
+// us with one thread walking a wave's winners, a round for each, and takes
+// 23.7; of 64 26.2 and 15.1, of 16 10.9 and 8.6.
+__device__ __forceinline__ void list_winners(const StepCtx& c, StepShared& sh, const WinnerList& l, uint32_t b0, uint32_t A) {
+    const LeoConfig& cfg = c.a->cfg;
+    const uint32_t nwaves = selecting_waves(c), wave = wave_index(), lane = __lane_id();
+    const uint32_t range = (cfg.block_count + nwaves - 1) / nwaves;
+    if (b0 > 0) {  // the waves with a place among these
+        l.owner[threadIdx.x] = 0u;
+        __syncthreads();
+        for (uint32_t wv = threadIdx.x; wv < nwaves; wv += kThreads) {
+            const uint32_t first = max(l.starts[wv], b0), end = min(l.starts[wv + 1], b0 + kThreads);
+            if (first < end) l.owner[first - b0] = wv + 1;
+        }
+        __syncthreads();
+    }
+    uint32_t owner = wave_incl_max_u32(l.owner[threadIdx.x]);
+    if (lane == kWaveSize - 1) sh.red[2][wave] = owner;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t w = 0; w + 1 < kWavesPerGroup; ++w)
+        if (w < wave) owner = max(owner, sh.red[2][w]);
+    const uint32_t f = b0 + threadIdx.x;
+    if (f < A) {
+        const uint32_t i = f - l.starts[owner - 1];
+        if (i > 0 || b0 > 0) {
+            const uint64_t at = static_cast<uint64_t>(owner - 1) * range * cfg.max_active_per_block + i;
+            l.ids[threadIdx.x] = ld(&c.d.range_winners[at]);
+            l.acts[threadIdx.x] = ld(&c.d.range_winner_act[at]);
+        }
+    }
+    __syncthreads();
 }
 
 // The readout runs in phase 3, beside the eligibility update, on the last
@@ -2998,8 +3057,7 @@ __device__ __forceinline__ uint32_t readout(const StepCtx& c, const StepParams& 
     uint32_t* ids = reinterpret_cast<uint32_t*>(step_lds);
     float* acts = reinterpret_cast<float*>(step_lds) + kThreads;
     float* ends = reinterpret_cast<float*>(step_lds) + 2 * kThreads;
-    uint32_t* starts = reinterpret_cast<uint32_t*>(step_lds) + 3 * kThreads;  // a list longer than kThreads
-    const uint32_t nwaves = selecting_waves(c), range = (cfg.block_count + nwaves - 1) / nwaves;
+    const WinnerList list{ids, acts, ids + 3 * kThreads, ids + 4 * kThreads};
     StepRecord LEO_GLOBAL& rec = d.records[step_index];
     if (end_thread) {
         rec.p_target = 0.0f;
@@ -3023,23 +3081,12 @@ __device__ __forceinline__ uint32_t readout(const StepCtx& c, const StepParams& 
     };
     for (uint32_t b0 = 0; b0 == 0 || b0 < A; b0 += kThreads) {
         ids[threadIdx.x] = 0u;
+        if (b0 == 0) list.owner[threadIdx.x] = 0u;
         __syncthreads();
         if (from_waves) {
-            if (b0 == 0) {
-                A = list_winners(c, sh, ids, acts);
-                if (A > kThreads) wave_starts(c, sh, starts, nwaves);
-            }
-            if (A > kThreads) {
-                uint32_t n = 0;
-                float act = 0.0f;
-                if (b0 + threadIdx.x < A) {
-                    (void)winner_key(d, starts, nwaves, range, cfg.block_count, cfg.max_active_per_block,
-                                     b0 + threadIdx.x, cfg.neuron_count, 0u, &n, &act);
-                    ids[threadIdx.x] = n;
-                    acts[threadIdx.x] = act;
-                }
-                __syncthreads();
-            }
+            bool more = true;
+            if (b0 == 0) A = list_first_winners(c, sh, list, &more);
+            if (more) list_winners(c, sh, list, b0, A);
         } else if (b0 + threadIdx.x < A) {
             const uint64_t at = static_cast<uint64_t>(rs) * cfg.max_active_global + b0 + threadIdx.x;
             ids[threadIdx.x] = ld(&d.ring_active[at]);

@@ -33,8 +33,8 @@ def _model(nb, blocks, fanout, limit, strength=1.0):
     return model
 
 
-def _step_us(model, run, steps):
-    """Best kernel time per step of five passes."""
+def _best(model, run, value):
+    """Smallest value of the kernel statistics of five passes."""
     from leo_amd.runtime import HipRuntime
 
     gpu = HipRuntime(model, device=0, max_lanes=1)
@@ -43,13 +43,17 @@ def _step_us(model, run, steps):
         for _ in range(5):
             gpu.kernel_stats(reset=True)
             run(gpu)
-            best = min(best, gpu.kernel_stats()["kernel_ms"] * 1e3 / steps)
+            best = min(best, value(gpu.kernel_stats()))
         return best
     finally:
         gpu.close()
 
 
 TEXT = story(5, 120)
+
+
+def _step_us(model, run, steps):
+    return _best(model, run, lambda stats: stats["kernel_ms"] * 1e3 / steps)
 
 
 def _frozen(gpu):
@@ -66,3 +70,23 @@ def test_ranking_many_candidates(require_gpu, nb, blocks, fanout, limit, most):
     dense = _step_us(_model(nb, blocks, fanout, limit), _frozen, len(TEXT))
     print(f"{blocks} blocks of {nb}: {none:.1f} us a step without candidates, {dense:.1f} us with", flush=True)
     assert dense < most * none
+
+
+# The readout's own time (phase 2 of the workgroup that selects nothing) with
+# two waves' winners in its list, against one winner a wave. A wave's winners
+# walked by one thread: 3.7 and 6.8 times; placed at once: 2.2 and 3.4.
+@pytest.mark.parametrize("winners,most", [(64, 2.9), (128, 4.8)])
+def test_reading_out_many_winners_of_a_wave(require_gpu, monkeypatch, winners, most):
+    monkeypatch.setenv("LEO_HIP_PHASE_PROFILE", "1")
+    monkeypatch.setenv("LEO_HIP_PROFILE_PART", "255")  # the last workgroup
+
+    def run(gpu):
+        gpu.evaluate([TEXT])
+
+    def work(stats):
+        return stats["phase_work_us"][2] / (len(TEXT) + 1)
+
+    one = _best(_model(1024, 2, 300, 1), run, work)
+    many = _best(_model(1024, 2, 300, winners), run, work)
+    print(f"{winners} winners a wave: readout {one:.1f} us with one, {many:.1f} us", flush=True)
+    assert many < most * one
