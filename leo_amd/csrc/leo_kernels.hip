@@ -3432,8 +3432,9 @@ __device__ __forceinline__ float inhibitory_step(const LeoConfig& cfg, float w, 
 // round. This ends the learning phase (3 us after the other workgroups at
 // 16,384 units and 32 dimensions; 5.2 us when the sums read weight and error
 // one output at a time): a learning step 36.2 -> 34.5 us there, 52.7 -> 51.1 at
-// a million units. Before that, with the projection loaded twice and a
-// division for every element's place, it took ~8 us.
+// a million units (32.7 and 47.1 with what came later). Before that, with the
+// projection loaded twice and a division for every element's place, it took
+// ~8 us.
 __device__ __forceinline__ void context_update(const StepCtx& c, const StepParams& sp, StepShared& sh,
                                                uint32_t step_index) {
     const LeoConfig& cfg = c.a->cfg;
@@ -3455,30 +3456,36 @@ __device__ __forceinline__ void context_update(const StepCtx& c, const StepParam
     const float old0 = threadIdx.x < cells ? ld(&d.p.ctx_emb[emb0]) : 0.0f;
     const uint32_t obs = threadIdx.x < count ? ld(&d.p.ctx_obs[sh.ctx_cell[threadIdx.x]]) : 0u;
     if (threadIdx.x == 0) ctl->ctx_out_dirty = 1;
+    // thread t: dimension t % kDims of outputs t / kDims, t / kDims + kOutputStep, ...;
+    // one 32-bit offset into the projection's buffer, which ends with the last
+    // output (seventeen 64-bit addresses kept from the loads to the stores
+    // spilled to scratch)
+    constexpr uint32_t kOutputStep = kThreads / kDims;
+    static_assert(kThreads % kDims == 0, "a thread keeps its dimension");
+    const __amdgpu_buffer_rsrc_t proj = coherent_rsrc(d.p.ctx_out, kOutputs * E * 4);
+    const uint32_t dim = threadIdx.x % kDims, o0 = threadIdx.x / kDims, step = kOutputStep * E * 4;
     for (uint32_t e0 = 0; e0 < E; e0 += kDims) {
+        const uint32_t e = e0 + dim, first = (o0 * E + e) * 4;
         float w[kEach];
 #pragma unroll
-        for (uint32_t k = 0; k < kEach; ++k) {
-            const uint32_t i = threadIdx.x + k * kThreads, o = i / kDims, e = e0 + i % kDims;
-            w[k] = o < kOutputs && e < E ? ld(&d.p.ctx_out[o * E + e]) : 0.0f;
-        }
+        for (uint32_t k = 0; k < kEach; ++k) w[k] = e < E ? ld4(proj, first + k * step) : 0.0f;
 #pragma unroll
         for (uint32_t k = 0; k < kEach; ++k) {
-            const uint32_t i = threadIdx.x + k * kThreads;
-            if (i < kOutputs * kDims) tile[i % kDims * kTileRow + i / kDims] = w[k] * sh.err[i / kDims];
+            const uint32_t o = o0 + k * kOutputStep;
+            if (o < kOutputs) tile[dim * kTileRow + o] = w[k] * sh.err[o];
         }
         __syncthreads();
         if (threadIdx.x < kDims && e0 + threadIdx.x < E)
             grad[e0 + threadIdx.x] = serial_sum_outputs(tile + threadIdx.x * kTileRow);
 #pragma unroll
         for (uint32_t k = 0; k < kEach; ++k) {
-            const uint32_t i = threadIdx.x + k * kThreads, o = i / kDims, e = e0 + i % kDims;
+            const uint32_t o = o0 + k * kOutputStep;
             if (o >= kOutputs || e >= E) continue;
             const float gradient = sh.err[o] * sh.latent[e];
             const float delta = bounded(-lr * strength * gradient, mu);
             const float updated = clampf(w[k] + delta, wmin, wmax);
             if (!finitef(updated)) set_step_error(ctl, kErrContextProjection, step_index);
-            d.p.ctx_out[o * E + e] = updated;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(updated), proj, first + k * step, 0, 0);
         }
         __syncthreads();
     }
@@ -4032,7 +4039,10 @@ __device__ __forceinline__ void lane_steps(const KernelArgs& args) {
 // The arguments live in device memory (read with scalar loads): a by-value
 // argument whose address is taken is copied to scratch.
 // Two waves per SIMD at the least: the cooperative capacity is planned for two
-// workgroups per CU, so the compiler keeps within 256 registers.
+// workgroups per CU, so the compiler keeps within 256 registers (the general
+// build needs 224, the profiled 234, the frozen-only 177, all without scratch;
+// a learning step with 84 bytes of scratch a lane took 34.3 us at 16,384 units
+// and 50.0 at a million, 32.7 and 47.1 without).
 __global__ void __launch_bounds__(kThreads, 2) leo_lane_steps(const KernelArgs* __restrict__ args) {
     lane_steps<false, false>(*args);
 }
