@@ -185,8 +185,6 @@ struct LaneControl {
     uint32_t ctx_count;
     uint32_t ctx_probes;
     uint32_t ctx_applied;
-    uint32_t ctx_slots[kMaxOrder];
-    float ctx_scales[kMaxOrder];
     uint32_t block_selected;
     uint32_t clipped;
     float pop_cutoff;
@@ -352,7 +350,6 @@ struct LaneDesc {
     float LEO_GLOBAL* logits;           // kOutStride
     float LEO_GLOBAL* probs;            // kOutStride
     float LEO_GLOBAL* errors;           // kOutStride
-    float LEO_GLOBAL* ctx_latent;       // E
     // change tracking bitmaps (ParameterChanges)
     uint32_t LEO_GLOBAL* ch_threshold;  // ceil(N/32)
     uint32_t LEO_GLOBAL* ch_rec;        // ceil(NS/32)

@@ -1059,17 +1059,13 @@ __device__ __forceinline__ void context_resolve(const StepCtx& c, const StepPara
             for (uint32_t t = 0; t < len; ++t) {
                 probes += sh.ctx_probes[t];
                 if (sh.ctx_slot[t] < 0) continue;
-                ctl->ctx_slots[count] = static_cast<uint32_t>(sh.ctx_slot[t]);
                 sh.ctx_cell[count] = static_cast<uint32_t>(sh.ctx_slot[t]);
                 scales[count] = sh.ctx_scale[t];
                 scale_sum += sh.ctx_scale[t];
                 count += 1;
             }
-            for (uint32_t i = 0; i < count; ++i) {
-                const float scale = scale_sum > 0.0f ? scales[i] / scale_sum : scales[i];
-                ctl->ctx_scales[i] = scale;
-                sh.ctx_weight[i] = scale;
-            }
+            for (uint32_t i = 0; i < count; ++i)
+                sh.ctx_weight[i] = scale_sum > 0.0f ? scales[i] / scale_sum : scales[i];
         }
         sh.ctx_cells = count;
         ctl->ctx_applied = enabled ? 1u : 0u;
@@ -2910,7 +2906,6 @@ __device__ __forceinline__ void context_logits(const StepCtx& c, StepShared& sh)
         for (uint32_t i = 0; i < kMaxOrder; ++i)
             if (i < cells && sh.ctx_weight[i] > 0.0f) v += emb[i] * sh.ctx_weight[i];
         sh.latent[e] = v;
-        d.ctx_latent[e] = v;
     }
     if (cells == 0) return;
     __syncthreads();
@@ -4200,7 +4195,6 @@ __global__ void __launch_bounds__(kThreads) leo_reset_lanes(KernelArgs args, uin
     }
     for (uint64_t i = t0; i < NI; i += ts) clear_record(d.in_trace, i);
     for (uint64_t i = t0; i < NI; i += ts) d.in_mark[i] = 0;
-    for (uint64_t i = t0; i < cfg.context_embedding_dim; i += ts) d.ctx_latent[i] = 0.0f;
     fill_u32(d.block_epoch, cfg.block_count, 0u, t0, ts);
     {
         // bucket counts and touched bits of every set (deliveries pending for

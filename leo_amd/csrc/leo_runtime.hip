@@ -500,7 +500,6 @@ void allocate_lane_state(Lane& lane, const Sizes& z, hipStream_t stream, uint32_
     size_t o_rt = l.add<float>(kTraceWords * z.ns), o_rm = l.add<uint8_t>(z.ns), o_rlist = l.add<uint32_t>(2 * z.ns);
     size_t o_it = l.add<float>(kTraceWords * z.ni), o_im = l.add<uint8_t>(z.ni), o_ilist = l.add<uint32_t>(2 * z.ni);
     size_t o_lg = l.add<float>(kOutStride), o_pr = l.add<float>(kOutStride), o_er = l.add<float>(kOutStride);
-    size_t o_lat = l.add<float>(std::max<uint64_t>(z.e, 1));
     size_t o_cth = l.add<uint32_t>(z.words(z.n)), o_crec = l.add<uint32_t>(z.words(z.ns)), o_cin = l.add<uint32_t>(z.words(z.ni));
     size_t o_cout = l.add<uint32_t>(z.words(z.n)), o_cctx = l.add<uint32_t>(z.words(z.slots));
     size_t o_prof = l.add<unsigned long long>(2 * kPhases);
@@ -544,7 +543,6 @@ void allocate_lane_state(Lane& lane, const Sizes& z, hipStream_t stream, uint32_
     d.logits = reinterpret_cast<float*>(b + o_lg);
     d.probs = reinterpret_cast<float*>(b + o_pr);
     d.errors = reinterpret_cast<float*>(b + o_er);
-    d.ctx_latent = reinterpret_cast<float*>(b + o_lat);
     d.ch_threshold = reinterpret_cast<uint32_t*>(b + o_cth);
     d.ch_rec = reinterpret_cast<uint32_t*>(b + o_crec);
     d.ch_in = reinterpret_cast<uint32_t*>(b + o_cin);
