@@ -2522,8 +2522,8 @@ void synchronize_host(LeoHipRuntime* h, LeoModelView& m) {
     const Sizes& z = h->z;
     const LaneDesc& d = h->canonical->desc;
     // at most this much packed data per download (a larger change set takes
-    // several)
-    constexpr size_t kPiece = size_t(64) << 20;
+    // several), and at most this much device scratch kept for the next call
+    constexpr size_t kPiece = size_t(64) << 20, kKeep = 2 * kPiece;
     constexpr size_t kCounts = 256;  // counts, then the lists' cursors, at the front of the scratch
     if (h->move_scratch.bytes < kCounts) h->move_scratch.allocate(kCounts);
     StagingRoute on_step_stream(h->staging, h->stream);
@@ -2554,18 +2554,20 @@ void synchronize_host(LeoHipRuntime* h, LeoModelView& m) {
     std::memcpy(flags, got_flags, sizeof(flags));
     std::memcpy(stale_flags, got_stale, sizeof(stale_flags));
     h->staging.drain();
-    // the lists on the device, then a region for one piece's values
+    // the lists on the device, then a region for one download's values (a set's
+    // values are up to three arrays)
     const uint64_t value_bytes[kChangeSets] = {4, 4, 4, kOutputs * 4, 12 + z.e * 4};
-    size_t list_at[kChangeSets], cursor = kCounts, largest = 0;
+    constexpr size_t kRounding = 3 * 256;
+    size_t list_at[kChangeSets], cursor = kCounts, values = 0;
     for (uint32_t i = 0; i < kChangeSets; ++i) {
         list_at[i] = cursor;
         cursor += PinnedStaging::rounded(count[i] * 4);
-        largest = std::max<size_t>(largest, std::min<size_t>(count[i] * value_bytes[i], kPiece + value_bytes[i]));
+        values += count[i] * value_bytes[i] + kRounding;
     }
     const size_t values_at = cursor;
-    const size_t need = values_at + kChangeSets * (largest + 4 * 256);
-    // with room for the sets' growth until tracking restarts
-    if (h->move_scratch.bytes < need) h->move_scratch.allocate(need + need / 2);
+    const size_t need = values_at + std::min(values, kPiece + kRounding);
+    // with room for the sets' growth until tracking restarts, as far as it is kept
+    if (h->move_scratch.bytes < need) h->move_scratch.allocate(std::max(need, std::min(need + need / 2, kKeep)));
     char* base = h->move_scratch.base;
     LEO_HIP_CHECK(hipMemsetAsync(base, 0, kCounts, h->stream));
     sets.count = reinterpret_cast<unsigned long long*>(base);
@@ -2617,37 +2619,37 @@ void synchronize_host(LeoHipRuntime* h, LeoModelView& m) {
             const size_t bytes = i == 4 ? keys_bytes + obs_bytes + PinnedStaging::rounded(n * z.e * 4)
                                         : PinnedStaging::rounded(n * value_bytes[i]);
             const size_t list_bytes = PinnedStaging::rounded(n * 4);
-            if (staged > 0 && (staged + bytes + list_bytes > kPiece || region + bytes > h->move_scratch.bytes)) {
+            if (staged > 0 && staged + bytes + list_bytes > kPiece) {
                 take_in();
                 staged = 0;
                 region = values_at;
             }
             if (staged == 0) h->staging.reserve(std::max(bytes + list_bytes, std::min<size_t>(kPiece, need)));
             const uint32_t* list = reinterpret_cast<const uint32_t*>(base + list_at[i]) + first;
-            char* values = base + region;
+            char* packed = base + region;
             if (i < 3) {
                 SparseMove mv{};
                 mv.tensor = const_cast<float*>(sources[i]);
                 mv.index = list;
-                mv.packed = reinterpret_cast<float*>(values);
+                mv.packed = reinterpret_cast<float*>(packed);
                 mv.count = n;
                 const uint64_t blocks = std::min<uint64_t>((n + kThreads - 1) / kThreads, 4096);
                 hipLaunchKernelGGL(leo_sparse_move, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, h->stream, mv);
             } else if (i == 3) {
-                const GatherRows g{h->canon.out_w, list, reinterpret_cast<float*>(values), n};
+                const GatherRows g{h->canon.out_w, list, reinterpret_cast<float*>(packed), n};
                 const uint64_t blocks = std::min<uint64_t>((n + kTransposeRows - 1) / kTransposeRows, 2048);
                 hipLaunchKernelGGL(leo_gather_rows, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, h->stream, g);
             } else {
-                const GatherSlots g{h->canon, list, n, static_cast<uint32_t>(z.e), reinterpret_cast<uint64_t*>(values),
-                                    reinterpret_cast<uint32_t*>(values + keys_bytes),
-                                    reinterpret_cast<float*>(values + keys_bytes + obs_bytes)};
+                const GatherSlots g{h->canon, list, n, static_cast<uint32_t>(z.e), reinterpret_cast<uint64_t*>(packed),
+                                    reinterpret_cast<uint32_t*>(packed + keys_bytes),
+                                    reinterpret_cast<float*>(packed + keys_bytes + obs_bytes)};
                 const uint64_t blocks = std::min<uint64_t>((n * z.e + kThreads - 1) / kThreads, 2048);
                 hipLaunchKernelGGL(leo_gather_slots, dim3(static_cast<uint32_t>(blocks)), dim3(kThreads), 0, h->stream, g);
             }
             LEO_HIP_CHECK(hipGetLastError());
             Piece piece{i, first, n, nullptr, nullptr};
             piece.index = h->staging.d2h(list, n * 4);
-            piece.values = h->staging.d2h(values, bytes);
+            piece.values = h->staging.d2h(packed, bytes);
             pieces.push_back(piece);
             staged += bytes + list_bytes;
             region += bytes;
@@ -2658,6 +2660,7 @@ void synchronize_host(LeoHipRuntime* h, LeoModelView& m) {
     if (flags[1] | stale_flags[1]) download(m.ctx_out, h->canon.ctx_out, kOutputs * z.e * 4, h->stream);
     clear_stale(h);
     sync(h->stream);
+    if (h->move_scratch.bytes > kKeep) h->move_scratch.release();
     m.generation = h->generation;
     m.parameter_revision = h->revision;
     m.statistics = h->stats;

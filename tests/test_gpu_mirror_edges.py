@@ -44,9 +44,8 @@ def test_mirror_follows_training(require_gpu):
         gpu.close()
 
 
-def test_mirror_of_more_rows_than_one_download(require_gpu):
-    from leo_amd.runtime import HipRuntime
-
+def _every_neuron_fires() -> Model:
+    """69,632 neurons whose output rows (68 MiB) all change in a learning step."""
     values = toml_values()
     n = 272 * 256
     values["model"].update(neuron_count=n, block_count=272, neurons_per_block=256, synapses_per_neuron=1,
@@ -63,6 +62,13 @@ def test_mirror_of_more_rows_than_one_download(require_gpu):
     model.in_weight[:] = np.float32(1.0)
     model.threshold[:] = np.float32(0.3)
     model.validate()
+    return model
+
+
+def test_mirror_of_more_rows_than_one_download(require_gpu):
+    from leo_amd.runtime import HipRuntime
+
+    model = _every_neuron_fires()
     mirror = model.copy()
     gpu = HipRuntime(model, device=0, max_lanes=1)
     try:
@@ -70,5 +76,35 @@ def test_mirror_of_more_rows_than_one_download(require_gpu):
         assert gpu.step(65, 66, native.TRAINING).active_neurons * 257 * 4 > (64 << 20)
         gpu.synchronize_model(mirror)
         assert_models_equal(mirror, gpu.model(), "every row")
+    finally:
+        gpu.close()
+
+
+
+def test_mirror_gives_scratch_back(require_gpu):
+    """A synchronisation keeps at most 128 MiB of device memory for the next."""
+    import ctypes
+
+    from leo_amd.runtime import HipRuntime
+
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    model = _every_neuron_fires()
+    mirror = model.copy()
+    gpu = HipRuntime(model, device=0, max_lanes=1)
+    try:
+        gpu.synchronize_model(mirror)
+        gpu.begin_document()
+        gpu.step(65, 66, native.TRAINING)
+        before = free_bytes()
+        gpu.synchronize_model(mirror)
+        kept = before - free_bytes()
+        print(f"{kept / 2**20:.0f} MiB kept", flush=True)
+        assert kept <= 130 << 20
     finally:
         gpu.close()
