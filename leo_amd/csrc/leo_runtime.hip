@@ -82,8 +82,10 @@ struct Arena {
     }
     void allocate(size_t n) {
         release();
+        char* p = nullptr;
+        LEO_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&p), std::max<size_t>(n, 256)));
+        base = p;  // a failed allocation leaves the arena empty, not of a size without memory
         bytes = n;
-        LEO_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&base), std::max<size_t>(n, 256)));
     }
 };
 
@@ -126,10 +128,12 @@ struct PinnedStaging {
         if (used + bytes <= capacity) return;
         drain();
         if (bytes <= capacity) return;
+        const size_t grown = std::max<size_t>({rounded(bytes), 2 * capacity, size_t(1) << 20});
         if (base) LEO_HIP_CHECK(hipHostFree(base));
         base = nullptr;
-        capacity = std::max<size_t>({rounded(bytes), 2 * capacity, size_t(1) << 20});
-        LEO_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&base), capacity, hipHostMallocDefault));
+        capacity = 0;  // a failed allocation leaves no room
+        LEO_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&base), grown, hipHostMallocDefault));
+        capacity = grown;
     }
     char* take(size_t bytes) {
         const size_t need = rounded(bytes);
