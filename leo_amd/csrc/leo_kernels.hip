@@ -3312,14 +3312,21 @@ __device__ __forceinline__ void phase_post(const StepCtx& c, const StepParams& s
 // first add, hands both on. Lanes 0-7 hold the even lines of A and the odd
 // lines of B, lanes 8-15 the others: every lane then takes line l from
 // register l. (The other lanes' sums at a stage are no row's and are not
-// used.) A batch costs one memory round and ~300 instructions whatever the
-// destinations number, and batches are dealt over every wave of the lane.
+// used.) A batch costs one memory round and ~300 instructions, most of them a
+// chain of adds, and batches are dealt over every wave of the lane: with many
+// batches a wave the chain bounds the phase, so that a wave sums two batches
+// at a time there.
 // With 64 rows a batch, staged through LDS line by line, a few hundred to a
 // thousand destinations occupied 8 to 23 waves of 64 to 128 for four memory
 // rounds. Post phase with signals, per step: 16,384 units, 506 destinations,
 // 64 waves: 7.2 us then, 4.8 now; a million units, ~1,000 destinations, 32
 // workgroups: 29% less; a 32-lane story pass at 131,072 units 17.8 -> 15.9 ms
-// (with the deep buckets' 1.1 ms).
+// (with the deep buckets' 1.1 ms). With one batch after the other (the next
+// one's rows loaded meanwhile) many destinations took longer than with 64 rows
+// a batch: 8,680 on 16 waves 97 us with 64 rows, 118 with eight, 95 with two
+// batches of eight at a time; on 64 waves 27.7, 31.7 and 25.6; 2,424 on 16
+// waves 29.2, 32.7 and 25.8; 808 on 128 waves (one batch a wave) 6.9, 4.3 and
+// 4.3.
 constexpr uint32_t kSignalRows = 8;
 constexpr uint32_t kSignalLines = kEndIndex / 32;  // 128-byte lines before the end-class weight
 
@@ -3331,78 +3338,125 @@ struct SignalRows {
 __device__ __forceinline__ uint32_t swap_halves(uint32_t v) {  // lanes 0-7 and 8-15 of each sixteen exchanged
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x128, 0xf, 0xf, false));
 }
-// `dst`: the destination of row lane / 8 (0 past the batch's end, `live` false).
-__device__ __forceinline__ void load_signal_rows(SignalRows& r, __amdgpu_buffer_rsrc_t rows, uint32_t dst, bool live) {
-    const uint32_t seg = __lane_id() & 7u;
-    const uint32_t other = swap_halves(dst);
-#pragma unroll
-    for (uint32_t l = 0; l < kSignalLines; ++l) r.line[l] = ld16_record(rows, (l & 1) ? other : dst, l * 128 + seg * 16);
+// `dst`: the destination of row lane / 8 (0 past the batch's end, `live`
+// false), `other` that of the row half a turn on.
+__device__ __forceinline__ void load_signal_line(SignalRows& r, __amdgpu_buffer_rsrc_t rows, uint32_t dst, uint32_t other,
+                                                 uint32_t l) {
+    r.line[l] = ld16_record(rows, (l & 1) ? other : dst, l * 128 + (__lane_id() & 7u) * 16);
+}
+__device__ __forceinline__ void end_signal_rows(SignalRows& r, __amdgpu_buffer_rsrc_t rows, uint32_t dst, uint32_t other,
+                                                bool live) {
     r.tail = ld4_record(rows, other, 4 * kEndIndex);
     r.dst_end = swap_halves(live ? dst : ~0u);
 }
-// The serial sums; lanes 7 and 15 of each sixteen return those of their dst_end.
-__device__ __forceinline__ float sum_signal_rows(const SignalRows& r, const f32x4 (&err)[kSignalLines], float err_end) {
-    float acc = 0.0f;
-    auto rotate = [](float v) {  // from the lane below, within sixteen
-        return __uint_as_float(static_cast<uint32_t>(
-            __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(v)), 0x121, 0xf, 0xf, false)));
-    };
+__device__ __forceinline__ void load_signal_rows(SignalRows& r, __amdgpu_buffer_rsrc_t rows, uint32_t dst, bool live) {
+    const uint32_t other = swap_halves(dst);
 #pragma unroll
-    for (uint32_t l = 0; l < kSignalLines; ++l) {
-        const float p0 = r.line[l].x * err[l].x, p1 = r.line[l].y * err[l].y;
-        const float p2 = r.line[l].z * err[l].z, p3 = r.line[l].w * err[l].w;
-#pragma unroll
-        for (uint32_t s = 0; s < 8; ++s) {
-            acc = rotate(acc) + p0;
-            acc += p1;
-            acc += p2;
-            acc += p3;
-        }
-    }
-    return acc + r.tail * err_end;
+    for (uint32_t l = 0; l < kSignalLines; ++l) load_signal_line(r, rows, dst, other, l);
+    end_signal_rows(r, rows, dst, other, live);
+}
+// Line l's 32 terms of the rows, added by the lane that holds the accumulator.
+struct SignalTerms {
+    float p[4];
+};
+__device__ __forceinline__ SignalTerms signal_terms(const SignalRows& r, const f32x4 (&err)[kSignalLines], uint32_t l) {
+    return {{r.line[l].x * err[l].x, r.line[l].y * err[l].y, r.line[l].z * err[l].z, r.line[l].w * err[l].w}};
+}
+__device__ __forceinline__ float signal_stage(float acc, const SignalTerms& t) {
+    // from the lane below, within sixteen
+    acc = __uint_as_float(static_cast<uint32_t>(
+              __builtin_amdgcn_update_dpp(0, static_cast<int>(__float_as_uint(acc)), 0x121, 0xf, 0xf, false))) + t.p[0];
+    acc += t.p[1];
+    acc += t.p[2];
+    acc += t.p[3];
+    return acc;
 }
 
 // The listed destinations' signals, the batches dealt round-robin over every
-// wave of the lane, the next batch's rows loaded while one is summed.
+// wave of the lane. A wave with several batches sums two at a time, one's adds
+// between the other's, and loads each line of the next two in the place of the
+// line just taken.
 __device__ __forceinline__ void phase_signals(const StepCtx& c, StepShared& sh) {
     const LaneDesc& d = c.d;
-    // one round: the errors, the destination count and this wave's first two
+    // one round: the errors, the destination count and this wave's first four
     // batches of the list (read before the count is known; entries past it
     // are masked below)
-    const uint32_t lane = __lane_id(), sub = lane >> 3;
+    const uint32_t lane = __lane_id(), sub = lane >> 3, seg = lane & 7u;
     const uint32_t stride = c.P * kWavesPerGroup * kSignalRows;
     const uint32_t N = c.a->cfg.neuron_count;
     uint32_t at = (wave_index() * c.P + c.part) * kSignalRows + sub;
     const uint32_t count = ld(&c.ctl->dest_count);
-    uint32_t dst = at < N ? ld(&d.dest_list[at]) : 0u;
-    uint32_t next = at + stride < N ? ld(&d.dest_list[at + stride]) : 0u;
+    auto listed = [&](uint32_t i) { return i < N ? ld(&d.dest_list[i]) : 0u; };
+    const uint32_t dst0 = listed(at), dst1 = listed(at + stride);
+    uint32_t next_a = listed(at + 2 * stride), next_b = listed(at + 3 * stride);
     for (uint32_t o = threadIdx.x; o < kOutputs; o += kThreads) sh.err[o] = ld(&d.errors[o]);
     __syncthreads();
     if (at - sub >= count) return;  // wave-uniform
     f32x4 err[kSignalLines];
 #pragma unroll
-    for (uint32_t l = 0; l < kSignalLines; ++l)
-        err[l] = reinterpret_cast<const f32x4*>(sh.err)[l * 8 + (lane & 7u)];
+    for (uint32_t l = 0; l < kSignalLines; ++l) err[l] = reinterpret_cast<const f32x4*>(sh.err)[l * 8 + seg];
     const float err_end = sh.err[kEndIndex];
-    // rows addressed by index (N records of kOutStride floats)
+    // rows addressed by index (N records of kOutStride floats); row 0 in the
+    // places past the list
     const __amdgpu_buffer_rsrc_t rows = record_rsrc(d.p.out_w, kOutStride * 4, N);
-    // two sets of rows in turn (a copy from one to the other would wait for
-    // the loads); true when a batch is left
-    SignalRows r0, r1;
-    load_signal_rows(r0, rows, at < count ? dst : 0u, at < count);
-    auto batch = [&](const SignalRows& cur, SignalRows& ahead) {
-        at += stride;
-        const bool more = at - sub < count;  // wave-uniform
-        if (more) {
-            load_signal_rows(ahead, rows, at < count ? next : 0u, at < count);
-            next = at + stride < N ? ld(&d.dest_list[at + stride]) : 0u;
-        }
-        const float sig = sum_signal_rows(cur, err, err_end);
-        if ((lane & 7u) == 7u && cur.dst_end != ~0u) d.learning_signal[cur.dst_end] = sig;
-        return more;
+    auto listed_row = [&](uint32_t i, uint32_t dst) { return i < count ? dst : 0u; };
+    // lanes 7 and 15 of each sixteen hold the sums
+    auto finish = [&](const SignalRows& r, float acc) {
+        const float sig = acc + r.tail * err_end;
+        if (seg == 7u && r.dst_end != ~0u) d.learning_signal[r.dst_end] = sig;
     };
-    while (batch(r0, r1) && batch(r1, r0)) {
+    auto sum_one = [&](const SignalRows& r) {
+        float acc = 0.0f;
+#pragma unroll
+        for (uint32_t l = 0; l < kSignalLines; ++l) {
+            const SignalTerms t = signal_terms(r, err, l);
+#pragma unroll
+            for (uint32_t s = 0; s < 8; ++s) acc = signal_stage(acc, t);
+        }
+        finish(r, acc);
+    };
+    SignalRows a, b;
+    load_signal_rows(a, rows, listed_row(at, dst0), at < count);
+    if (at - sub + stride >= count) {  // (wave-uniform, like the conditions below)
+        sum_one(a);
+        return;
     }
+    load_signal_rows(b, rows, listed_row(at + stride, dst1), at + stride < count);
+    // sums a and b; `more`: loads the next two batches into them
+    auto sum_two = [&](auto more) {
+        uint32_t dst[2] = {0, 0}, other[2] = {0, 0};
+        if (more) {
+            dst[0] = listed_row(at + 2 * stride, next_a);
+            dst[1] = listed_row(at + 3 * stride, next_b);
+            next_a = listed(at + 4 * stride);
+            next_b = listed(at + 5 * stride);
+            other[0] = swap_halves(dst[0]);
+            other[1] = swap_halves(dst[1]);
+        }
+        float acc_a = 0.0f, acc_b = 0.0f;
+#pragma unroll
+        for (uint32_t l = 0; l < kSignalLines; ++l) {
+            const SignalTerms ta = signal_terms(a, err, l), tb = signal_terms(b, err, l);
+            if (more) {
+                load_signal_line(a, rows, dst[0], other[0], l);
+                load_signal_line(b, rows, dst[1], other[1], l);
+            }
+#pragma unroll
+            for (uint32_t s = 0; s < 8; ++s) {
+                acc_a = signal_stage(acc_a, ta);
+                acc_b = signal_stage(acc_b, tb);
+            }
+        }
+        finish(a, acc_a);
+        finish(b, acc_b);
+        if (more) {
+            end_signal_rows(a, rows, dst[0], other[0], at + 2 * stride < count);
+            end_signal_rows(b, rows, dst[1], other[1], at + 3 * stride < count);
+        }
+    };
+    for (; at - sub + 2 * stride < count; at += 2 * stride) sum_two(std::true_type{});
+    if (at - sub + stride < count) sum_two(std::false_type{});
+    else sum_one(a);
 }
 
 // ---------------------------------------------------------------------------

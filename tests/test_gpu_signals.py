@@ -43,3 +43,12 @@ def test_signal_batches_match_oracle(require_gpu, oracle, fanout):
         assert_models_equal(gpu.model(), cpu.model(), f"fanout {fanout}")
     finally:
         gpu.close()
+
+
+@pytest.mark.parametrize("fanout", [32, 33, 63, 64, 65, 96, 97, 128, 136, 161, 500, 1000])
+def test_many_batches_a_wave_match_oracle(require_gpu, oracle, monkeypatch, fanout):
+    """One workgroup: four waves of eight destinations a batch, so that a wave
+    takes one, two, an odd and an even number of batches, whole and ragged."""
+    monkeypatch.setenv("LEO_HIP_CANONICAL_WGS", "1")
+    monkeypatch.setenv("LEO_HIP_WGS_PER_LANE", "1")
+    test_signal_batches_match_oracle(require_gpu, oracle, fanout)
