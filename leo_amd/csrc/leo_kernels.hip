@@ -470,7 +470,6 @@ constexpr uint32_t kInjectAhead = kBucketSets - 1;
 struct alignas(16) StepShared {
     float err[kOutStride];                                      // errors / logits
     float aux[kOutStride + kThreads];                           // exps, latent, gradient
-    uint32_t scan[kThreads];
     uint32_t red[3][kWavesPerGroup];
     float redf[2][kWavesPerGroup];
     // context resolution (one thread per order)
@@ -2416,24 +2415,27 @@ __device__ __forceinline__ float frozen_prologue(const StepCtx& c, StepShared& s
 
 // First active-list position of each selecting wave's winners (block order,
 // runtime.rs:1010-1013) into starts[0..nwaves], starts[nwaves] = the total;
-// by the whole workgroup (the running scan uses sh.scan).
+// by the whole workgroup. (Scanned through LDS, two barriers a doubling, it held
+// up every step of a binding cap: 19.8 us a frozen step at 249,344 units, 23.7
+// at 32,768; 18.9 and 22.7 now.)
 __device__ __forceinline__ uint32_t wave_starts(const StepCtx& c, StepShared& sh, uint32_t* starts, uint32_t nwaves) {
+    const uint32_t wave = wave_index();
     uint32_t running = 0;
     for (uint32_t base = 0; base < nwaves; base += kThreads) {
         const uint32_t wv = base + threadIdx.x;
         const uint32_t v = wv < nwaves ? ld(&wave_totals(c.d, c.tick)[wv]) : 0;
-        sh.scan[threadIdx.x] = v;
+        const uint32_t incl = wave_incl_scan_u32(v);
+        if (__lane_id() == kWaveSize - 1) sh.red[0][wave] = incl;
         __syncthreads();
-        for (uint32_t off = 1; off < kThreads; off <<= 1) {
-            const uint32_t add = threadIdx.x >= off ? sh.scan[threadIdx.x - off] : 0;
-            __syncthreads();
-            sh.scan[threadIdx.x] += add;
-            __syncthreads();
+        uint32_t at = running + incl - v;
+#pragma unroll
+        for (uint32_t w = 0; w < kWavesPerGroup; ++w) {
+            const uint32_t total = sh.red[0][w];
+            at += w < wave ? total : 0u;
+            running += total;
         }
-        if (wv < nwaves) starts[wv] = running + sh.scan[threadIdx.x] - v;
-        const uint32_t chunk_total = sh.scan[kThreads - 1];
+        if (wv < nwaves) starts[wv] = at;
         __syncthreads();
-        running += chunk_total;
     }
     if (threadIdx.x == 0) starts[nwaves] = running;
     __syncthreads();
