@@ -1283,8 +1283,10 @@ __device__ __forceinline__ void deep_ranks(const Key* keys, uint32_t cnt, const 
 // Latency-bound: the wave that owns a hub ends the lane's phase. With 131,072
 // units and power-law targets (1,876 deliveries a step, hubs of 70-200) a
 // frozen step took 22.6 us with ranks counted and entries broadcast through
-// lane reads up to 128 entries and a radix sort above, and takes 17.1 us; at
-// 256 entries the ranking is ~1,000 compares a lane, still under the radix
+// lane reads up to 128 entries and a radix sort above, and takes 17.1 us. With
+// the line to the radix sort at 128 entries instead of 256 a 400-byte prompt
+// there takes 6.38 ms instead of 6.04 and 32 evaluated stories 5.27 instead of
+// 4.95: up to 256 the ranking (~1,000 compares a lane) stays under the radix
 // sort's three passes over memory, and four entries per lane is what the 2 KB
 // stage holds.
 __device__ __forceinline__ float deep_ranked_sum(const KernelArgs& a, const uint64_t LEO_GLOBAL* set_base,
@@ -1673,14 +1675,15 @@ __device__ __forceinline__ uint32_t count_smaller(const uint64_t* keys, uint32_t
 // (deep_ranks), those of several blocks sorted first and eight keys a round
 // (count_smaller). Frozen steps with ~230 candidates in a wave's one block of
 // 256 took 91 us when each comparison was a dependent pair of LDS reads, 37
-// with eight keys a round after listing in neuron order, and take 29; with
-// ~910 in a block of 1,024 they took 1,015, 268 and take 182.
+// with eight keys a round after listing in neuron order, and take 27; with
+// ~910 in a block of 1,024 they took 1,015, 268 and take 142.
 // Bound by the chain of dependent instructions and memory rounds of one wave
 // per SIMD, not by bandwidth. Listing in neuron order took a scan and LDS
 // writes per row of 64 words, and block starts, counts and ranks went through
 // LDS: 470 frozen and 32 learning steps at a million units (33 blocks, ~22
-// touched neurons a wave) took 7.46 ms then and 7.07 now, a batch at 1,024
-// units (one block, ~84 touched neurons a wave) 74 ms then and 62 now.
+// touched neurons a wave) took 7.46 ms of step-kernel time then and 7.07 after
+// (whole calls 8.66 and 8.31), a batch at 1,024 units (one block, ~84 touched
+// neurons a wave) 74 ms and 62 (88.7 and 77.5).
 // `keep_bits`: a trace step leaves the bitmap words set for its eligibility
 // update (the learning phase clears them from the touched list). `pi` is the
 // population inhibition the previous tick left; `post_pending` that the
@@ -2806,8 +2809,13 @@ __device__ __forceinline__ void eligibility_list(const StepCtx& c, float LEO_GLO
 }
 
 // Slots per lane and iteration for a list of n slots over gstride threads:
-// four when two a thread would take a second iteration, else two (a wider
-// iteration costs a lane with one or two slots more than it saves).
+// four when two a thread would take a second iteration, else two. Whole calls
+// against two everywhere and against four past eight slots a thread: a learned
+// document of a dense 1,280-unit model 18.6, 18.0 and 17.9 ms, 24 story lanes
+// at 131,072 units 13.2, 12.2 and 12.0, one of 200 bytes at 16,384 units 7.28,
+// 7.23 and 7.05-7.24; at a million units and with thousands of slots a thread
+// within 1% (four where one or two are left would add their loads and shuffles
+// for nothing).
 template <class F>
 __device__ __forceinline__ void eligibility_width(uint32_t n, uint32_t gstride, F&& walk) {
     if (n > 2u * gstride) walk(std::integral_constant<uint32_t, 4>{});
