@@ -3001,8 +3001,9 @@ __device__ __forceinline__ uint32_t list_first_winners(const StepCtx& c, StepSha
 // last one with a first place up to here (a maximum scan over `owner`; waves
 // without winners have none), and one memory round brings every winner that
 // is not there yet. The readout of 128 winners in each of two waves took 46.9
-// us with one thread walking a wave's winners, a round for each, and takes
-// 23.7; of 64 26.2 and 15.1, of 16 10.9 and 8.6.
+// us with one thread walking a wave's winners, a round for each, and 23.7 so;
+// of 64 26.2 and 15.1, of 16 10.9 and 8.6 (15.8 and 11.1 for 128 and 64 with
+// the readout's sum of the end class since).
 __device__ __forceinline__ void list_winners(const StepCtx& c, StepShared& sh, const WinnerList& l, uint32_t b0, uint32_t A) {
     const LeoConfig& cfg = c.a->cfg;
     const uint32_t nwaves = selecting_waves(c), wave = wave_index(), lane = __lane_id();

@@ -63,7 +63,8 @@ def _frozen(gpu):
 
 # Frozen steps with nearly every neuron of a wave's one block a candidate,
 # against the same deliveries with none. With one dependent pair of LDS reads a
-# comparison 46 and 7.5 times; with independent reads 8.4 and 2.4.
+# comparison 46 and 7.5 times; with independent reads 8.4 and 2.4 (6.5 and 2.2 with
+# runs of blocks planned by one scan).
 @pytest.mark.parametrize("nb,blocks,fanout,limit,most", [(1024, 2, 1900, 64, 20.0), (256, 4, 1000, 16, 4.2)])
 def test_ranking_many_candidates(require_gpu, nb, blocks, fanout, limit, most):
     none = _step_us(_model(nb, blocks, fanout, limit, 0.001), _frozen, len(TEXT))
@@ -74,8 +75,9 @@ def test_ranking_many_candidates(require_gpu, nb, blocks, fanout, limit, most):
 
 # The readout's own time (phase 2 of the workgroup that selects nothing) against
 # that of two winners. Two waves' winners, 64 and 128 each: walked by one thread
-# a wave 3.7 and 6.8 times; placed at once 2.2 and 3.4. 1,024 winners: with the
-# end class summed one LDS read a term 11.6 times, sixteen a round 7.1.
+# a wave 3.7 and 6.8 times; placed at once 2.2 and 3.4 (1.6 and 2.3 with the end
+# class summed sixteen terms a round). 1,024 winners: with the end class summed
+# one LDS read a term 11.6 times, sixteen a round 7.1.
 @pytest.mark.parametrize("nb,blocks,fanout,winners,most",
                          [(1024, 2, 300, 64, 2.9), (1024, 2, 300, 128, 4.8), (256, 64, 1500, 16, 9.1)])
 def test_reading_out_many_winners(require_gpu, monkeypatch, nb, blocks, fanout, winners, most):
